@@ -95,8 +95,8 @@ void release_scene(Ctx& c) {
     BuildScratch& b = c.scratch;
     b.keys.release(); b.keys_alt.release(); b.vals.release(); b.vals_alt.release(); b.sort_tmp.release();
     b.prim_lo.release(); b.prim_hi.release(); b.bparent.release(); b.bchild.release(); b.brange.release();
-    b.bnode_lo.release(); b.bnode_hi.release(); b.bflag.release(); b.queue_a.release(); b.queue_b.release();
-    b.counters.release(); b.bounds.release(); b.node_depth.release();
+    b.bnode_lo.release(); b.bnode_hi.release(); b.bflag.release(); b.elem.release();
+    b.counters.release(); b.bounds.release();
     c.h_instances.clear();
     c.h_meshes.clear();
     c.num_lights = 0;

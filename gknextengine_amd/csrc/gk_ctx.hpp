@@ -125,10 +125,9 @@ struct BuildScratch {
     DevBuf<uint2> brange;                 // [first, last] of each internal node
     DevBuf<float4> bnode_lo, bnode_hi;    // internal node boxes (w = cost / prim count)
     DevBuf<uint32_t> bflag;               // bottom-up arrival counters
-    DevBuf<uint32_t> queue_a, queue_b;    // top-down collapse work queues (pairs)
-    DevBuf<uint32_t> counters;            // [0] wide node count [1] queue size [2] next queue size
+    DevBuf<uint32_t> elem;                // binary subtree of each wide node (top-down collapse)
+    DevBuf<uint32_t> counters;            // wide nodes per level
     DevBuf<float> bounds;                 // scene centroid bounds (6 floats as ordered ints)
-    DevBuf<uint32_t> node_depth;
 };
 
 // ------------------------------------------------------------------ context

@@ -279,3 +279,34 @@ def test_closest_hit_does_not_depend_on_ray_order(device):
     assert _u32(res[0][i:i + 1, 3])[0] == 168450, res[0][i]
     for k in (1, 2):
         assert np.array_equal(_u32(res[k]), _u32(res[0])), int((_u32(res[k]) != _u32(res[0])).any(1).sum())
+
+
+# sizes around the builder's steps: one leaf, a work-group of 256 leaves in the bottom-up pass,
+# the 4096 primitives that one work-group collapses, and several work-groups
+@pytest.mark.parametrize("n", [1, 2, 4, 5, 255, 256, 257, 4095, 4096, 4097, 20000])
+def test_build_sizes_trace_as_the_oracle(device, n):
+    """Random triangle soups (with repeated triangles, so that Morton codes tie): the closest
+    hits of a built tree equal the oracle's bit for bit, and every triangle is reached."""
+    rng = np.random.default_rng(n)
+    s = gk.SceneData()
+    v = rng.uniform(-1, 1, (n, 1, 3)) + rng.normal(0, 0.15, (n, 3, 3))
+    v[n // 2:n // 2 + n // 8] = v[:n // 8]
+    s.add_mesh(v.reshape(-1, 3), np.arange(3 * n, dtype=np.uint32).reshape(-1, 3))
+    s.materials = [scenes.Bricks(n_side=1).scene.materials[0]]
+    s.add_instance(0)
+    rays = scenes.random_rays(4000, -1.5, 1.5, seed=n, tmin=1e-3, tmax=1000.0)
+    with gk.Context(16, 16) as ctx:
+        ctx.upload(s)
+        h, _ = gpu_trace(ctx, rays, device)
+        stats = ctx.bvh_stats()
+        # a ray straight at each triangle's centre, ending just behind it, meets something
+        c = v.mean(1)
+        nrm = np.cross(v[:, 1] - v[:, 0], v[:, 2] - v[:, 0])
+        nrm /= np.linalg.norm(nrm, axis=1, keepdims=True)
+        at = np.zeros((n, 8), np.float32)
+        at[:, :3], at[:, 4:7], at[:, 7] = c - 0.01 * nrm, nrm, 0.02
+        ho, _ = gpu_trace(ctx, at, device, any_hit=True)
+    assert stats.blas_nodes <= max(1, n) and stats.sah_cost > 0
+    o, _ = po.OracleScene(s).trace(rays)
+    assert np.array_equal(_u32(h), _u32(o))
+    assert np.all(_u32(ho[:, 3]) == 1)
