@@ -21,8 +21,9 @@
 //
 // Kernels
 //   k_conv    forward convolution (also the input gradient, with flipped weights)
-//   k_wgrad   weight gradient: dW[cout][k] = sum_pixels g[pixel][cout] * im2col[k][pixel]
-//   k_pool / k_pool_bwd / k_upsum / k_relu_mask / k_loss / k_adam / k_wflip / k_pack /
+//   k_wgrad   weight gradient: dW[cout][k] = sum_pixels g[pixel][cout] * im2col[k][pixel], in
+//             partial rows that k_wgrad_sum adds
+//   k_pool / k_pool_bwd / k_upsum / k_loss / k_adam / k_wflip / k_pack /
 //   k_unpack / k_frame_input: elementwise and reductions
 #include <hip/hip_runtime.h>
 
@@ -62,10 +63,17 @@ __device__ inline bf16x8 pack8(const uint16_t (&v)[8]) {
     return __builtin_bit_cast(bf16x8, make_uint4(uint32_t(v[0]) | (uint32_t(v[1]) << 16), uint32_t(v[2]) | (uint32_t(v[3]) << 16),
                                                  uint32_t(v[4]) | (uint32_t(v[5]) << 16), uint32_t(v[6]) | (uint32_t(v[7]) << 16)));
 }
-__device__ inline void st4(uint16_t* p, float a, float b, float c, float d) {
-    *reinterpret_cast<uint2*>(p) = make_uint2(uint32_t(f2bf(a)) | (uint32_t(f2bf(b)) << 16),
-                                              uint32_t(f2bf(c)) | (uint32_t(f2bf(d)) << 16));
+// two bf16 gradients where the two bf16 activations are > 0 (sign bit clear and not +0), else 0
+__device__ inline uint32_t relu_mask2(uint32_t gw, uint32_t yw) {
+    const uint32_t lo = ((yw & 0x8000u) == 0u && (yw & 0x7fffu) != 0u) ? 0xffffu : 0u;
+    const uint32_t hi = ((yw & 0x80000000u) == 0u && (yw & 0x7fff0000u) != 0u) ? 0xffff0000u : 0u;
+    return gw & (lo | hi);
 }
+__device__ inline uint2 relu_mask4(uint2 g, uint2 y) { return make_uint2(relu_mask2(g.x, y.x), relu_mask2(g.y, y.y)); }
+__device__ inline uint2 bf4(float a, float b, float c, float d) {
+    return make_uint2(uint32_t(f2bf(a)) | (uint32_t(f2bf(b)) << 16), uint32_t(f2bf(c)) | (uint32_t(f2bf(d)) << 16));
+}
+__device__ inline void st4(uint16_t* p, float a, float b, float c, float d) { *reinterpret_cast<uint2*>(p) = bf4(a, b, c, d); }
 
 // ---------------------------------------------------------------- convolution
 struct ConvK {
@@ -75,6 +83,7 @@ struct ConvK {
     uint16_t* out;      // channels [0, split), stride split
     uint16_t* out2;     // channels [split, cout), stride cout - split
     float* outf;        // when set: channels 0..3 as one float4 per pixel
+    const uint16_t* mask;  // MASK: out is zero where this tensor (out's shape) is not > 0
     uint32_t ca, cb, cin, a_up;
     uint32_t W, H, tiles_y;
     uint32_t kpad, ktap;  // ktap = 9 * cin
@@ -101,7 +110,7 @@ __host__ __device__ inline uint32_t conv_weight_bytes(uint32_t mt, uint32_t kpad
     return mt * 16u * (kpad / 8u + 1u) * 16u;
 }
 
-template <int MT, int MODE>
+template <int MT, int MODE, bool MASK>
 __global__ __launch_bounds__(256) void k_conv(ConvK K) {
     constexpr bool STAGE = MODE >= 1;
     extern __shared__ uint4 tile[];
@@ -247,7 +256,9 @@ __global__ __launch_bounds__(256) void k_conv(ConvK K) {
             if (K.outf) {
                 if (co == 0) *reinterpret_cast<float4*>(K.outf + px * 4) = make_float4(v0, v1, v2, v3);
             } else if (co < split) {
-                st4(K.out + px * split + co, v0, v1, v2, v3);
+                uint2 v = bf4(v0, v1, v2, v3);
+                if (MASK) v = relu_mask4(v, *reinterpret_cast<const uint2*>(K.mask + px * split + co));
+                *reinterpret_cast<uint2*>(K.out + px * split + co) = v;
             } else {
                 st4(K.out2 + px * (cout - split) + (co - split), v0, v1, v2, v3);
             }
@@ -992,116 +1003,259 @@ __global__ __launch_bounds__(256) void k_convs1(ConvS K) {
 }
 
 // ---------------------------------------------------------------- weight gradient
+// dW[co][tap][ci] = sum over pixels p of g[p][co] * in[p + tap][ci]: a GEMM whose reduction
+// runs along pixels, which NHWC does not keep consecutive for a channel. A work-group copies
+// a tile of 32 pixels x 4 nrg rows of both tensors into LDS as it lies in memory (16-byte
+// global-to-LDS loads, no registers in between), and the operands are read with the LDS
+// transpose load, which hands a lane 4 pixels of its channel: 16 lanes address 4 pixels x 16
+// channels, lane i gets channel i. A lane's 8 reduction slots are pixels 4 q .. 4 q + 3 and
+// 16 + 4 q .. (q = lane / 16) in both operands. Of the two operands the input is shifted by dx
+// (its tile has a halo column on each side) and the gradient by dy (a halo row above and
+// below), so a wave reads three input operands and MT new gradient operands per 9 MT MFMAs.
+// A wave owns 16 input channels, MT * 16 output channels and 4 rows; the ncw waves side by
+// side share the gradient tile, nrg groups of them take different rows.
+//
+// LDS banks: 8 consecutive pixels of one 16-channel segment (32 bytes) are read in a cycle
+// pair and have to cover the 8 segments of 256 bytes. With n segments per pixel they do when
+// n is odd; for n = 2^k m the segment's position is XORed with the pixel's bits 3-k .. 2
+// (WgradSwz), by choosing which 16 bytes a staging lane loads.
+//
+// Work-group (b, i, j) of a layer sums tiles [b T / S, (b + 1) T / S) in its registers, then
+// writes one partial row of the layer's gradient; k_wgrad_sum adds the S rows in order, in
+// double, so that no atomics are needed and the gradient is the same on every run.
+// Bound: the latency of a tile's loads, one work-group per CU (above). The 8 x 256 x 256
+// training step's twelve launches and their sum: 2180 -> 290 us (with operands gathered 2
+// bytes at a time from memory and 32-bit atomics into the gradient before).
 struct WgradK {
     const uint16_t* a;
     const uint16_t* b;
     const uint16_t* g;  // gradient at the convolution output (after the ReLU mask), [pixel][cout]
-    float* dw;          // [cout][kpad], accumulated
+    float* part;        // [S][cout][kpad]
     uint32_t ca, cb, cin, a_up;
-    uint32_t W, H, rows, rows_per_block;
-    uint32_t kpad, ktap, cout, bias;
+    uint32_t W, H, ntx, nty, tiles;  // tiles = images x nty x ntx
+    uint32_t kpad, cout;
+    uint32_t ncw, nrg;  // 16-channel input groups and 4-row groups of a work-group's waves
 };
 
-// One work-group = 4 waves over rows_per_block image rows (the GEMM's reduction), MT*16
-// output channels and NT*16 columns k. Each wave reduces its own rows and adds its tile
-// to dw with atomics. Operands are gathered 2 bytes at a time (the reduction runs along
-// pixels, which are not contiguous in NHWC for a fixed channel).
-template <int MT, int NT>
-__global__ __launch_bounds__(256) void k_wgrad(WgradK K) {
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+constexpr uint32_t kWgCols = 32;                 // pixels of a tile row (one MFMA's reduction)
+constexpr uint32_t kWgRows = 4;                  // rows of a wave
+constexpr uint32_t kWgXCols = 40;                // staged input columns x0 - 1 .. (34 used; a multiple of 8)
+struct WgradSwz {
+    uint32_t shift, mask;
+    __host__ __device__ explicit WgradSwz(uint32_t n)
+        : shift(n % 8u == 0u ? 0u : (n % 4u == 0u ? 1u : (n % 2u == 0u ? 2u : 3u))),
+          mask(n % 8u == 0u ? 7u : (n % 4u == 0u ? 3u : (n % 2u == 0u ? 1u : 0u))) {}
+    __host__ __device__ uint32_t operator()(uint32_t seg, uint32_t pixel) const {
+        return seg ^ ((pixel >> shift) & mask);
+    }
+};
+// LDS bytes of the two tiles
+__host__ __device__ inline uint32_t wg_xbytes(uint32_t ncw, uint32_t nrg) { return kWgRows * nrg * kWgXCols * ncw * 32u; }
+inline uint32_t wg_lds_bytes(uint32_t mt, uint32_t ncw, uint32_t nrg) {
+    const uint32_t tiles = wg_xbytes(ncw, nrg) + (kWgRows * nrg + 2u) * kWgCols * mt * 32u;
+    const uint32_t sums = nrg > 1u ? ncw * 10u * mt * 1024u : 0u;  // one row group's accumulators
+    return tiles > sums ? tiles : sums;
+}
+
+__device__ uint4 wg_zero;  // source of the tiles' pixels outside the image (zero from the load on)
+
+// 16 bytes per lane from src into LDS at dst (wave-uniform) + 16 * lane
+__device__ inline void load_to_lds(const void* src, char* dst) {
+    __builtin_amdgcn_global_load_lds(reinterpret_cast<const __attribute__((address_space(1))) void*>(reinterpret_cast<uintptr_t>(src)),
+                                     (__attribute__((address_space(3))) void*)(dst), 16, 0, 0);
+}
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4* lds_s16x4;
+// two transpose loads at LDS byte addresses p0, p1
+__device__ inline bf16x8 read_tr(uint32_t p0, uint32_t p1) {
+    union { s16x4 h[2]; bf16x8 v; } u;
+    u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(p0));
+    u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(p1));
+    return u.v;
+}
+
+template <int MT>
+__global__ __launch_bounds__(512) void k_wgrad(WgradK K) {
+    extern __shared__ uint4 wg_lds[];
+    char* const xs = reinterpret_cast<char*>(wg_lds);
+    char* const gs = xs + wg_xbytes(K.ncw, K.nrg);
+    const uint32_t xs0 = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)(xs)));
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wv = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)));
+    const uint32_t ciw = wv % K.ncw, rg = wv / K.ncw, nw = K.ncw * K.nrg;
     const int W = int(K.W), H = int(K.H);
-    const int co0 = blockIdx.z * (MT * 16);
-    const int kt0 = blockIdx.y * (NT * 16);
-    const int kg = (lane >> 4) * 8;
-    const int cin = int(K.cin), ca = int(K.ca), cb = int(K.cb), cout = int(K.cout);
-    // column of this lane in each B tile: kind 0 zero, 1 data, 2 bias
-    int kind[NT], dxj[NT], dyj[NT], cij[NT];
+    const uint32_t th = kWgRows * K.nrg;
+    const uint32_t ci0 = blockIdx.y * K.ncw * 16u, co0 = blockIdx.z * (MT * 16u);
+    const uint32_t xrow = kWgXCols * K.ncw * 32u;          // bytes of a staged input row
+    constexpr uint32_t grow = kWgCols * MT * 32u;          // and of a gradient row
+    const WgradSwz xsw(K.ncw), gsw(MT);
+    // the input tile is th * 40 * 2 ncw = 5 * 64 nw units of 16 bytes: five per thread, whose
+    // row, column and channel (of the unit that the swizzle puts there) are the same in every tile
+    uint32_t xu[5];
 #pragma unroll
-    for (int j = 0; j < NT; ++j) {
-        const int kcol = kt0 + j * 16 + (lane & 15);
-        kind[j] = 0;
-        dxj[j] = dyj[j] = cij[j] = 0;
-        if (kcol < int(K.ktap)) {
-            const int tap = kcol / cin;
-            cij[j] = kcol - tap * cin;
-            dyj[j] = tap / 3 - 1;
-            dxj[j] = tap - (tap / 3) * 3 - 1;
-            kind[j] = 1;
-        } else if (kcol == int(K.ktap) && K.bias) {
-            kind[j] = 2;
+    for (uint32_t k = 0; k < 5; ++k) {
+        const uint32_t u = (k * nw + wv) * 64u + lane;
+        const uint32_t pix = u / (2u * K.ncw), in = u - pix * (2u * K.ncw);
+        const uint32_t row = pix / kWgXCols, col = pix - row * kWgXCols;
+        xu[k] = row | (col << 8) | ((xsw(in >> 1, col) * 16u + (in & 1u) * 8u) << 16);
+    }
+    // operand addresses: lane i of a 16-lane group addresses pixel i / 4, channels 4 (i % 4) ..
+    const uint32_t pc = 4u * (lane >> 4) + ((lane & 15u) >> 2), cb8 = (lane & 3u) * 8u;
+    uint32_t xa[3][2], ga_off[MT][2];
+#pragma unroll
+    for (uint32_t h = 0; h < 2; ++h) {
+#pragma unroll
+        for (uint32_t x3 = 0; x3 < 3; ++x3) {  // dx + 1: staged column 0 is x0 - 1
+            const uint32_t col = pc + 16u * h + x3;
+            xa[x3][h] = (col * K.ncw + xsw(ciw, col)) * 32u + cb8;
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < MT; ++i) ga_off[i][h] = ((pc + 16u * h) * MT + gsw(i, pc + 16u * h)) * 32u + cb8;
+    }
+    f32x4 acc[9][MT], accb[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        accb[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < 9; ++t) acc[t][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    const bool with_bias = blockIdx.y == 0 && ciw == 0;
+    const uint32_t t0 = uint32_t((uint64_t(blockIdx.x) * K.tiles) / gridDim.x);
+    const uint32_t t1 = uint32_t((uint64_t(blockIdx.x + 1) * K.tiles) / gridDim.x);
+    for (uint32_t t = t0; t < t1; ++t) {
+        const uint32_t img = t / (K.ntx * K.nty), tr = t - img * K.ntx * K.nty;
+        const int y0 = int((tr / K.ntx) * th), x0 = int((tr % K.ntx) * kWgCols);
+        __syncthreads();  // the last tile's operands have been read
+#pragma unroll
+        for (uint32_t k = 0; k < 5; ++k) {
+            // selects instead of branches: the five loads are issued one behind the other
+            const int y = y0 + int(xu[k] & 0xffu), col = int((xu[k] >> 8) & 0xffu), x = x0 - 1 + col;
+            const uint32_t c = ci0 + (xu[k] >> 16);
+            const bool first = c < K.ca;
+            const uint32_t up = first ? K.a_up : 0u;  // half resolution: W, H, x and y are even there
+            const uint32_t row = img * (K.H >> up) + (uint32_t(y) >> up);
+            const uint64_t pix = uint64_t(row) * (K.W >> up) + (uint32_t(x) >> up);
+            const uint16_t* src = (first ? K.a : K.b) + pix * (first ? K.ca : K.cb) + (first ? c : c - K.ca);
+            const bool ok = x >= 0 && x < W && y < H && col < int(kWgCols) + 2;
+            src = ok ? src : reinterpret_cast<const uint16_t*>(&wg_zero);
+            load_to_lds(src, xs + (k * nw + wv) * 1024u);
+        }
+        for (uint32_t q = wv; q < (th + 2u) * MT; q += nw) {  // 64 units of the gradient tile
+            const uint32_t u = q * 64u + lane;
+            const uint32_t pix = u / (2u * MT), in = u - pix * (2u * MT);
+            const uint32_t row = pix / kWgCols, col = pix - row * kWgCols;
+            const uint32_t c = co0 + gsw(in >> 1, col) * 16u + (in & 1u) * 8u;
+            const int y = y0 - 1 + int(row), x = x0 + int(col);
+            const uint16_t* src = K.g + ((uint64_t(img) * K.H + uint32_t(y)) * K.W + uint32_t(x)) * K.cout + c;
+            src = y >= 0 && y < H && x < W ? src : reinterpret_cast<const uint16_t*>(&wg_zero);
+            load_to_lds(src, gs + q * 1024u);
+        }
+        __builtin_amdgcn_s_waitcnt(0);  // the tiles are in LDS
+        __syncthreads();
+        // input row q meets gradient rows q - dy, dy = 1, 0, -1: staged rows q, q + 1, q + 2
+        uint32_t xr = xs0 + rg * kWgRows * xrow, gr = xs0 + wg_xbytes(K.ncw, K.nrg) + rg * kWgRows * grow;
+        // opaque here, so that the operand addresses are formed in the loop (one add each)
+        // instead of being kept for every row across tiles
+        asm volatile("" : "+s"(xr), "+s"(gr));
+        bf16x8 ga[kWgRows + 2][MT];
+#pragma unroll
+        for (uint32_t q = 0; q < kWgRows + 2; ++q) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i) ga[q][i] = read_tr(gr + q * grow + ga_off[i][0], gr + q * grow + ga_off[i][1]);
+            if (q < 2) continue;
+            // a row's operands are not read before the row above is done: three rows of
+            // gradient operands stay in registers, not six
+            __builtin_amdgcn_sched_barrier(0);
+            const uint32_t row = q - 2;
+            bf16x8 bx[3];
+#pragma unroll
+            for (int x3 = 0; x3 < 3; ++x3) bx[x3] = read_tr(xr + row * xrow + xa[x3][0], xr + row * xrow + xa[x3][1]);
+#pragma unroll
+            for (int j = 0; j < 3; ++j)  // dy = 1 - j
+#pragma unroll
+                for (int x3 = 0; x3 < 3; ++x3)
+#pragma unroll
+                    for (int i = 0; i < MT; ++i)
+                        acc[3 * (2 - j) + x3][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            ga[row + j][i], bx[x3], acc[3 * (2 - j) + x3][i], 0, 0, 0);
+        }
+        if (with_bias) {
+            // the bias column's input is 1; apart from the rows above, whose accumulators then
+            // stay in place
+            const bf16x8 ones = __builtin_bit_cast(bf16x8, make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
+#pragma unroll 1
+            for (uint32_t q = 1; q <= kWgRows; ++q)
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+                    accb[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        read_tr(gr + q * grow + ga_off[i][0], gr + q * grow + ga_off[i][1]), ones, accb[i], 0, 0, 0);
         }
     }
-    f32x4 acc[MT][NT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const uint32_t r_end = min(K.rows, (blockIdx.x + 1) * K.rows_per_block);
-    for (uint32_t r = blockIdx.x * K.rows_per_block + wv; r < r_end; r += 4) {
-        const int img = int(r / K.H), y = int(r - uint32_t(img) * K.H);
-        const size_t px0 = size_t(img) * H * W;
-        const size_t pxa0 = size_t(img) * (H >> 1) * (W >> 1);
-        for (int x0 = 0; x0 < W; x0 += 32) {
-            bf16x8 af[MT];
+    // the row groups' accumulators are added through LDS, one group at a time
+    f32x4* const sums = reinterpret_cast<f32x4*>(wg_lds) + size_t(ciw) * (10 * MT) * 64;
+    for (uint32_t k = 1; k < K.nrg; ++k) {
+        __syncthreads();
+        if (rg == k) {
 #pragma unroll
             for (int i = 0; i < MT; ++i) {
-                const uint16_t* gp = K.g + (px0 + size_t(y) * W) * cout + co0 + i * 16 + (lane & 15);
-                uint16_t v[8];
+                sums[(9 * MT + i) * 64 + lane] = accb[i];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int xx = x0 + kg + e;
-                    v[e] = xx < W ? gp[size_t(xx) * cout] : uint16_t(0);
-                }
-                af[i] = pack8(v);
+                for (int t = 0; t < 9; ++t) sums[(t * MT + i) * 64 + lane] = acc[t][i];
             }
-            bf16x8 bfr[NT];
+        }
+        __syncthreads();
+        if (rg == 0) {
 #pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                uint16_t v[8];
-                const int sy = y + dyj[j];
-                const bool yin = sy >= 0 && sy < H;
+            for (int i = 0; i < MT; ++i) {
+                accb[i] += sums[(9 * MT + i) * 64 + lane];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int xx = x0 + kg + e;
-                    uint16_t val = 0;
-                    if (xx < W) {
-                        if (kind[j] == 2) {
-                            val = 0x3f80u;
-                        } else if (kind[j] == 1) {
-                            const int sx = xx + dxj[j];
-                            if (yin && sx >= 0 && sx < W) {
-                                const int c = cij[j];
-                                if (c < ca)
-                                    val = K.a_up ? K.a[(pxa0 + size_t(sy >> 1) * (W >> 1) + (sx >> 1)) * ca + c]
-                                                 : K.a[(px0 + size_t(sy) * W + sx) * ca + c];
-                                else
-                                    val = K.b[(px0 + size_t(sy) * W + sx) * cb + (c - ca)];
-                            }
-                        }
-                    }
-                    v[e] = val;
-                }
-                bfr[j] = pack8(v);
+                for (int t = 0; t < 9; ++t) acc[t][i] += sums[(t * MT + i) * 64 + lane];
             }
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int j = 0; j < NT; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bfr[j], acc[i][j], 0, 0, 0);
         }
     }
+    if (rg != 0) return;
+    float* const out = K.part + size_t(blockIdx.x) * K.cout * K.kpad;
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j) {
-            const int kcol = kt0 + j * 16 + (lane & 15);
+        for (int e = 0; e < 4; ++e) {
+            float* row = out + size_t(co0 + i * 16 + (lane >> 4) * 4 + e) * K.kpad;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int co = co0 + i * 16 + (lane >> 4) * 4 + e;
-                const float v = acc[i][j][e];
-                if (v != 0.f) unsafeAtomicAdd(K.dw + size_t(co) * K.kpad + kcol, v);
-            }
+            for (int t = 0; t < 9; ++t) row[t * K.cin + ci0 + ciw * 16u + (lane & 15)] = acc[t][i][e];
+            if (with_bias && (lane & 15) == 0) row[9u * K.cin] = accb[i][e];
         }
+}
+
+// The layers' gradients from their partial rows: 64 parameters per work-group, 16 threads
+// (four parameters each) x 16 interleaved rows; the padding behind the bias column is zero.
+struct WgradSum {
+    const float* part[kLayers];
+    uint32_t rows[kLayers], first[kLayers], kpad[kLayers], ktap[kLayers];  // first: parameter offset
+    uint32_t end;
+};
+__global__ __launch_bounds__(256) void k_wgrad_sum(WgradSum K, float* __restrict__ grad) {
+    __shared__ double red[16][64];
+    const uint32_t p0 = blockIdx.x * 64u;  // a layer's parameters are a multiple of 512
+    uint32_t l = 0;
+#pragma unroll
+    for (uint32_t k = 1; k < kLayers; ++k) l = p0 >= K.first[k] ? k : l;
+    const uint32_t size = (l + 1 < kLayers ? K.first[l + 1] : K.end) - K.first[l];
+    const uint32_t q = threadIdx.x & 15u, s0 = threadIdx.x >> 4;
+    const float* src = K.part[l] + (p0 - K.first[l]) + q * 4u;
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
+    for (uint32_t s = s0; s < K.rows[l]; s += 16u) {
+        const float4 x = *reinterpret_cast<const float4*>(src + size_t(s) * size);
+        v[0] += double(x.x); v[1] += double(x.y); v[2] += double(x.z); v[3] += double(x.w);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) red[s0][q * 4u + e] = v[e];
+    __syncthreads();
+    if (threadIdx.x < 64u) {
+        double a = 0.0;
+        for (int k = 0; k < 16; ++k) a += red[k][threadIdx.x];
+        const uint32_t col = (p0 - K.first[l] + threadIdx.x) % K.kpad[l];
+        grad[p0 + threadIdx.x] = col <= K.ktap[l] ? float(a) : 0.f;
+    }
 }
 
 // ---------------------------------------------------------------- elementwise
@@ -1133,8 +1287,9 @@ __global__ void k_pool(const uint16_t* s, uint16_t* p, uint32_t nimg, uint32_t H
     st4(o + 4, 0.25f * acc[4], 0.25f * acc[5], 0.25f * acc[6], 0.25f * acc[7]);
 }
 
-// gS (H x W) += gP (H/2 x W/2) / 4 broadcast to each 2x2 block
-__global__ void k_pool_bwd(const uint16_t* gp, uint16_t* gs, uint32_t nimg, uint32_t H, uint32_t W, uint32_t c) {
+// gS (H x W) += gP (H/2 x W/2) / 4 broadcast to each 2x2 block, then the ReLU mask of the
+// activation act that gS is the gradient of
+__global__ void k_pool_bwd(const uint16_t* gp, const uint16_t* act, uint16_t* gs, uint32_t nimg, uint32_t H, uint32_t W, uint32_t c) {
     const uint32_t Ho = H / 2, Wo = W / 2, g8 = c / 8;
     const size_t t = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (t >= size_t(nimg) * Ho * Wo * g8) return;
@@ -1152,19 +1307,22 @@ __global__ void k_pool_bwd(const uint16_t* gp, uint16_t* gs, uint32_t nimg, uint
         const size_t pi = (size_t(img) * H + 2 * y + (d >> 1)) * W + 2 * x + (d & 1);
         uint16_t* o = gs + pi * c + grp * 8;
         const uint4 u = *reinterpret_cast<const uint4*>(o);
+        const uint4 y4 = *reinterpret_cast<const uint4*>(act + pi * c + grp * 8);
         const uint32_t s4[4] = {u.x, u.y, u.z, u.w};
         float r[8];
         for (int e = 0; e < 4; ++e) {
             r[2 * e] = __uint_as_float(s4[e] << 16) + q[2 * e];
             r[2 * e + 1] = __uint_as_float(s4[e] & 0xffff0000u) + q[2 * e + 1];
         }
-        st4(o, r[0], r[1], r[2], r[3]);
-        st4(o + 4, r[4], r[5], r[6], r[7]);
+        const uint2 a = relu_mask4(bf4(r[0], r[1], r[2], r[3]), make_uint2(y4.x, y4.y));
+        const uint2 b = relu_mask4(bf4(r[4], r[5], r[6], r[7]), make_uint2(y4.z, y4.w));
+        *reinterpret_cast<uint4*>(o) = make_uint4(a.x, a.y, b.x, b.y);
     }
 }
 
-// gA (H/2 x W/2) = sum of gUp over each 2x2 block (adjoint of nearest upsampling)
-__global__ void k_upsum(const uint16_t* gu, uint16_t* ga, uint32_t nimg, uint32_t H, uint32_t W, uint32_t c) {
+// gA (H/2 x W/2) = sum of gUp over each 2x2 block (adjoint of nearest upsampling), then the
+// ReLU mask of the activation act that gA is the gradient of
+__global__ void k_upsum(const uint16_t* gu, const uint16_t* act, uint16_t* ga, uint32_t nimg, uint32_t H, uint32_t W, uint32_t c) {
     const uint32_t Ho = H / 2, Wo = W / 2, g8 = c / 8;
     const size_t t = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (t >= size_t(nimg) * Ho * Wo * g8) return;
@@ -1181,28 +1339,10 @@ __global__ void k_upsum(const uint16_t* gu, uint16_t* ga, uint32_t nimg, uint32_
             acc[2 * e + 1] += __uint_as_float(w4[e] & 0xffff0000u);
         }
     }
-    uint16_t* o = ga + po * c + grp * 8;
-    st4(o, acc[0], acc[1], acc[2], acc[3]);
-    st4(o + 4, acc[4], acc[5], acc[6], acc[7]);
-}
-
-// g = y > 0 ? g : 0, 8 bf16 per thread
-__global__ void k_relu_mask(uint16_t* g, const uint16_t* y, size_t n8) {
-    const size_t t = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= n8) return;
-    uint4 gv = reinterpret_cast<uint4*>(g)[t];
-    const uint4 yv = reinterpret_cast<const uint4*>(y)[t];
-    auto m = [](uint32_t gw, uint32_t yw) {
-        // bf16 > 0: sign bit clear and not +0
-        const uint32_t lo = ((yw & 0x8000u) == 0u && (yw & 0x7fffu) != 0u) ? 0xffffu : 0u;
-        const uint32_t hi = ((yw & 0x80000000u) == 0u && (yw & 0x7fff0000u) != 0u) ? 0xffff0000u : 0u;
-        return gw & (lo | hi);
-    };
-    gv.x = m(gv.x, yv.x);
-    gv.y = m(gv.y, yv.y);
-    gv.z = m(gv.z, yv.z);
-    gv.w = m(gv.w, yv.w);
-    reinterpret_cast<uint4*>(g)[t] = gv;
+    const uint4 y4 = *reinterpret_cast<const uint4*>(act + po * c + grp * 8);
+    const uint2 a = relu_mask4(bf4(acc[0], acc[1], acc[2], acc[3]), make_uint2(y4.x, y4.y));
+    const uint2 b = relu_mask4(bf4(acc[4], acc[5], acc[6], acc[7]), make_uint2(y4.z, y4.w));
+    *reinterpret_cast<uint4*>(ga + po * c + grp * 8) = make_uint4(a.x, a.y, b.x, b.y);
 }
 
 // features (n x h x w x 10, FP32) -> X (n x hp x wp x 16, BF16): log(1+radiance), albedo,
@@ -1247,32 +1387,32 @@ __global__ void k_unpack_display(const float* Y, ushort4* out, uint32_t h, uint3
                             display_encode(b, paper_white, hdr != 0u), 1.f);
 }
 
-// loss = sum (z - log(1+t))^2 / (3 n h w); g = d loss / d z as BF16 (16 channels)
+// loss = sum (z - log(1+t))^2 / (3 n h w); g = d loss / d z as BF16 (16 channels). Work-groups
+// take several pixels per thread: with one each, 2048 double atomics on one address took most
+// of the kernel (8 x 256 x 256: 31 -> 15 us)
 __global__ __launch_bounds__(256) void k_loss(const float* Y, const float* target, uint16_t* g, size_t npx,
                                               float inv_count, double* loss) {
-    __shared__ float red[256];
-    const size_t t = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    float l = 0.f;
-    if (t < npx) {
+    __shared__ double red[256];
+    double l = 0.0;
+    const float s = 2.f * inv_count;
+    for (size_t t = size_t(blockIdx.x) * blockDim.x + threadIdx.x; t < npx; t += size_t(gridDim.x) * blockDim.x) {
         const float4 z = reinterpret_cast<const float4*>(Y)[t];
         const float d0 = z.x - log1pf(fmaxf(target[3 * t], 0.f));
         const float d1 = z.y - log1pf(fmaxf(target[3 * t + 1], 0.f));
         const float d2 = z.z - log1pf(fmaxf(target[3 * t + 2], 0.f));
-        l = d0 * d0 + d1 * d1 + d2 * d2;
-        uint16_t* o = g + t * 16;
-        const float s = 2.f * inv_count;
-        st4(o, s * d0, s * d1, s * d2, 0.f);
-        st4(o + 4, 0.f, 0.f, 0.f, 0.f);
-        st4(o + 8, 0.f, 0.f, 0.f, 0.f);
-        st4(o + 12, 0.f, 0.f, 0.f, 0.f);
+        l += double(d0 * d0 + d1 * d1 + d2 * d2);
+        const uint2 v = bf4(s * d0, s * d1, s * d2, 0.f);
+        uint4* o = reinterpret_cast<uint4*>(g + t * 16);
+        o[0] = make_uint4(v.x, v.y, 0u, 0u);
+        o[1] = make_uint4(0u, 0u, 0u, 0u);
     }
     red[threadIdx.x] = l;
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (int(threadIdx.x) < s) red[threadIdx.x] += red[threadIdx.x + s];
+    for (int w = 128; w > 0; w >>= 1) {
+        if (int(threadIdx.x) < w) red[threadIdx.x] += red[threadIdx.x + w];
         __syncthreads();
     }
-    if (threadIdx.x == 0) atomicAdd(loss, double(red[0]) * double(inv_count));
+    if (threadIdx.x == 0) atomicAdd(loss, red[0] * double(inv_count));
 }
 
 __global__ void k_adam(float* w, float* m, float* v, const float* g, uint16_t* w16, size_t n, float lr, float b1,
@@ -1408,6 +1548,7 @@ struct gk_unet {
     DevBuf<float> w32, m, v, grad;
     DevBuf<uint16_t> w16, wt16;
     DevBuf<double> loss;
+    DevBuf<float> wpart;               // partial rows of the weight gradients (training)
     uint64_t step = 0;
     TensorInfo tinfo[T_COUNT] = {};
     DevBuf<uint16_t> t[T_COUNT];
@@ -1504,38 +1645,55 @@ static uint32_t max_lds_per_block() {
 // of dynamic LDS the kernel's limit is raised first (the level-3 decoder convolution of the
 // 32-channel network stages 86 KB: 76.8 -> 57.9 us at 1080p), and a refused raise keeps the
 // direct loads
-template <int MT>
-void launch_conv_t(const ConvK& K, uint32_t nimg, hipStream_t st) {
+constexpr uint32_t kConvOnePerCu = 192;  // of 256 CUs
+template <int MT, bool MASK>
+void launch_conv_m(const ConvK& K, uint32_t nimg, hipStream_t st) {
     const dim3 grid((K.W + 15) / 16, K.tiles_y * nimg, K.cout / (MT * 16));
     const uint32_t bytes = conv_tile_bytes(K.ca, K.cb, K.a_up);
     const uint32_t wbytes = conv_weight_bytes(MT, K.kpad);
     bool stage = (K.W % 2u) == 0u && (K.H % 2u) == 0u && bytes <= max_lds_per_block();
-    // weights join the tile while both stay within 64 KB (two or more work-groups per CU)
-    if (stage && bytes + wbytes <= 65536u) {
-        k_conv<MT, 2><<<grid, 256, bytes + wbytes, st>>>(K);
-        return;
+    // weights join the tile while both stay within 64 KB (two or more work-groups per CU), or
+    // whatever fits a CU when the launch has fewer work-groups than CUs: the K loop then waits
+    // for no weight load (8 x 256 x 256, input gradients of levels 3 and 4: 21 -> 15 us; at 256
+    // work-groups the copy of the weights costs more than it saves, 21 -> 28 us)
+    const uint32_t groups = grid.x * grid.y * grid.z;
+    const uint32_t room = groups <= kConvOnePerCu ? max_lds_per_block() : 65536u;
+    if (stage && bytes + wbytes <= room) {
+        const void* fn = reinterpret_cast<const void*>(&k_conv<MT, 2, MASK>);
+        if (bytes + wbytes <= 65536u ||
+            hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes + wbytes)) == hipSuccess) {
+            k_conv<MT, 2, MASK><<<grid, 256, bytes + wbytes, st>>>(K);
+            return;
+        }
+        (void)hipGetLastError();
     }
     if (stage && bytes > 65536u) {
-        const void* fn = reinterpret_cast<const void*>(&k_conv<MT, 1>);
+        const void* fn = reinterpret_cast<const void*>(&k_conv<MT, 1, MASK>);
         if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)) != hipSuccess) {
             (void)hipGetLastError();
             stage = false;
         }
     }
-    if (stage) k_conv<MT, 1><<<grid, 256, bytes, st>>>(K);
-    else k_conv<MT, 0><<<grid, 256, 0, st>>>(K);
+    if (stage) k_conv<MT, 1, MASK><<<grid, 256, bytes, st>>>(K);
+    else k_conv<MT, 0, MASK><<<grid, 256, 0, st>>>(K);
+}
+template <int MT>
+void launch_conv_t(const ConvK& K, uint32_t nimg, hipStream_t st) {
+    if (K.mask) launch_conv_m<MT, true>(K, nimg, st);
+    else launch_conv_m<MT, false>(K, nimg, st);
 }
 
 int launch_conv(ConvK K, uint32_t nimg, hipStream_t st) {
     // the most output channels per work-group that still give at least 256 work-groups (the
     // coarse levels have 40 to 135 pixel tiles: one work-group per tile left most CUs idle),
     // unless the staged input tile is above 64 KB (then every extra work-group stages it
-    // again: the level-3 decoder convolution's 86 KB tile ran at 72 us split three ways
-    // against 58 us whole)
+    // again: the level-3 decoder convolution's 86 KB tile at 1080p, 135 tiles, ran at 72 us
+    // split three ways against 58 us whole) and there is a tile for every other CU (at 32
+    // tiles, the 8 x 256 x 256 batch: 60 us whole, 31 us split six ways)
     const uint32_t nm = K.cout / 16;
     K.tiles_y = (K.H + 15) / 16;
     const uint32_t tiles = ((K.W + 15) / 16) * K.tiles_y * nimg;
-    const bool split = conv_tile_bytes(K.ca, K.cb, K.a_up) <= 65536u;
+    const bool split = conv_tile_bytes(K.ca, K.cb, K.a_up) <= 65536u || tiles < 128u;
     int mt = 1;
     for (int c = 8; c >= 1; --c)
         if (nm % uint32_t(c) == 0u && (!split || tiles * (nm / uint32_t(c)) >= 256u)) {
@@ -1646,29 +1804,60 @@ int launch_convs(const gk_unet_layer& L, ConvS K, uint32_t nimg, bool pool, int 
     return kNoShape;
 }
 
-template <int MT, int NT>
-void launch_wgrad_t(const WgradK& K, hipStream_t st) {
-    const dim3 grid((K.rows + K.rows_per_block - 1) / K.rows_per_block, K.kpad / (NT * 16), K.cout / (MT * 16));
-    k_wgrad<MT, NT><<<grid, 256, 0, st>>>(K);
+// How the weight gradient of a layer is split. MT output-channel tiles per wave: at most 3,
+// whose accumulators leave two waves per SIMD (4 spill: the 8 x 256 x 256 step 1.14 against
+// 1.11 ms). As many 16-channel input groups side by side as divide the input (at most 8 waves,
+// each reading the same gradient tile), row groups so that a work-group has about 4 waves, and
+// along the pixels enough work-groups for one per CU: a partial row is as large as the layer's
+// gradient, so more rows cost more to write and add than they hide (step at 192, 256, 384 and
+// 512 work-groups: 1.25, 1.11, 1.16, 1.16 ms). kWgradPart floats of partials at most.
+constexpr size_t kWgradPart = size_t(1) << 24;
+struct WgradPlan {
+    uint32_t mt, ncw, nrg, tiles, rows;  // rows: work-groups along the pixels = partial rows
+};
+WgradPlan plan_wgrad(const gk_unet_layer& L, uint32_t nimg, uint32_t W, uint32_t H) {
+    WgradPlan p{};
+    const uint32_t nm = L.cout / 16u, nc = (L.cin_a + L.cin_b) / 16u;
+    for (uint32_t m = 3; m >= 1 && !p.mt; --m)
+        if (nm % m == 0u) p.mt = m;
+    for (uint32_t m = 8; m >= 1 && !p.ncw; --m)
+        if (nc % m == 0u) p.ncw = m;
+    p.nrg = p.ncw == 1u ? 4u : (p.ncw == 2u ? 2u : 1u);
+    const uint32_t th = kWgRows * p.nrg;
+    p.tiles = nimg * ((H + th - 1u) / th) * ((W + kWgCols - 1u) / kWgCols);
+    const uint32_t across = (nm / p.mt) * (nc / p.ncw);
+    const size_t row = size_t(L.cout) * L.kpad;
+    size_t rows = std::max(1u, 256u / across);
+    rows = std::min<size_t>(rows, std::max<size_t>(1u, kWgradPart / row));
+    p.rows = uint32_t(std::min<size_t>(rows, p.tiles));
+    return p;
 }
 
-int launch_wgrad(WgradK K, hipStream_t st) {
-    const uint32_t nm = K.cout / 16, nn = K.kpad / 16;
-    const int mt = nm % 4u == 0u ? 4 : (nm % 3u == 0u ? 3 : (nm % 2u == 0u ? 2 : 1));
-    const int nt = nn % 4u == 0u ? 4 : 2;
-    K.rows_per_block = 16;
-    switch (mt * 10 + nt) {
-        case 44: launch_wgrad_t<4, 4>(K, st); break;
-        case 42: launch_wgrad_t<4, 2>(K, st); break;
-        case 34: launch_wgrad_t<3, 4>(K, st); break;
-        case 32: launch_wgrad_t<3, 2>(K, st); break;
-        case 24: launch_wgrad_t<2, 4>(K, st); break;
-        case 22: launch_wgrad_t<2, 2>(K, st); break;
-        case 14: launch_wgrad_t<1, 4>(K, st); break;
-        default: launch_wgrad_t<1, 2>(K, st); break;
-    }
+template <int MT>
+int launch_wgrad_t(const WgradK& K, const WgradPlan& p, hipStream_t st) {
+    const uint32_t bytes = wg_lds_bytes(MT, p.ncw, p.nrg);
+    const void* fn = reinterpret_cast<const void*>(&k_wgrad<MT>);
+    if (bytes > max_lds_per_block()) return GK_ERR_LIMIT;
+    if (bytes > 65536u) GK_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)));
+    const dim3 grid(p.rows, K.cin / (16u * p.ncw), K.cout / (16u * MT));
+    k_wgrad<MT><<<grid, 64u * p.ncw * p.nrg, bytes, st>>>(K);
     GK_HIP(hipGetLastError());
     return GK_OK;
+}
+
+int launch_wgrad(WgradK K, const WgradPlan& p, hipStream_t st) {
+    K.ncw = p.ncw;
+    K.nrg = p.nrg;
+    const uint32_t th = kWgRows * p.nrg;
+    K.ntx = (K.W + kWgCols - 1u) / kWgCols;
+    K.nty = (K.H + th - 1u) / th;
+    K.tiles = p.tiles;
+    switch (p.mt) {
+        case 4: return launch_wgrad_t<4>(K, p, st);
+        case 3: return launch_wgrad_t<3>(K, p, st);
+        case 2: return launch_wgrad_t<2>(K, p, st);
+        default: return launch_wgrad_t<1>(K, p, st);
+    }
 }
 
 const uint16_t* tp(gk_unet& n, int i) { return i == kNone ? nullptr : n.t[i].ptr; }
@@ -1787,11 +1976,30 @@ int pack_input(gk_unet& n, const float* in, uint32_t nimg, uint32_t h, uint32_t 
 int backward(gk_unet& n, const float* target, uint32_t nimg, uint32_t h, uint32_t w, float* grad) {
     hipStream_t st = n.ctx->stream;
     const size_t npx = size_t(nimg) * h * w;
-    k_fill<<<nblk(n.nparam), 256, 0, st>>>(grad, n.nparam);
-    GK_HIP(hipGetLastError());
+    // every layer's partial rows have a place of their own; one launch adds them at the end
+    WgradPlan plan[kLayers];
+    WgradSum sum{};
+    size_t floats = 0;
+    for (uint32_t l = 0; l < kLayers; ++l) {
+        const gk_unet_layer& L = n.L[l];
+        plan[l] = plan_wgrad(L, nimg, w >> L.level, h >> L.level);
+        floats += size_t(plan[l].rows) * L.cout * L.kpad;
+    }
+    if (n.wpart.count < floats) GK_HIP(n.wpart.resize(floats));
+    floats = 0;
+    for (uint32_t l = 0; l < kLayers; ++l) {
+        const gk_unet_layer& L = n.L[l];
+        sum.part[l] = n.wpart.ptr + floats;
+        sum.rows[l] = plan[l].rows;
+        sum.first[l] = uint32_t(L.offset);
+        sum.kpad[l] = L.kpad;
+        sum.ktap[l] = 9u * (L.cin_a + L.cin_b);
+        floats += size_t(plan[l].rows) * L.cout * L.kpad;
+    }
+    sum.end = uint32_t(n.nparam);
     k_fill<<<1, 32, 0, st>>>(reinterpret_cast<float*>(n.loss.ptr), 2);
     GK_HIP(hipGetLastError());
-    k_loss<<<nblk(npx), 256, 0, st>>>(n.y32.ptr, target, n.t[G_Y].ptr, npx, 1.f / float(3 * npx), n.loss.ptr);
+    k_loss<<<std::min(nblk(npx), 512u), 256, 0, st>>>(n.y32.ptr, target, n.t[G_Y].ptr, npx, 1.f / float(3 * npx), n.loss.ptr);
     GK_HIP(hipGetLastError());
     for (int l = int(kLayers) - 1; l >= 0; --l) {
         const gk_unet_layer& L = n.L[l];
@@ -1799,28 +2007,22 @@ int backward(gk_unet& n, const float* target, uint32_t nimg, uint32_t h, uint32_
         const uint32_t lw = w >> L.level, lh = h >> L.level;
         const uint32_t cin = L.cin_a + L.cin_b;
         uint16_t* g = n.t[S.gout].ptr;
-        if (L.relu) {
-            const size_t n8 = size_t(nimg) * lh * lw * L.cout / 8;
-            k_relu_mask<<<nblk(n8), 256, 0, st>>>(g, n.t[S.out].ptr, n8);
-            GK_HIP(hipGetLastError());
-        }
+        // the kernel that wrote g last applied the ReLU mask of this layer's output: the input
+        // gradient of the layer after it (post 0), k_upsum (1) or k_pool_bwd (2)
         WgradK Wk{};
         Wk.a = tp(n, S.a);
         Wk.b = tp(n, S.b);
         Wk.g = g;
-        Wk.dw = grad + L.offset;
+        Wk.part = const_cast<float*>(sum.part[l]);
         Wk.ca = L.cin_a;
         Wk.cb = L.cin_b;
         Wk.cin = cin;
         Wk.a_up = L.up;
         Wk.W = lw;
         Wk.H = lh;
-        Wk.rows = nimg * lh;
         Wk.kpad = L.kpad;
-        Wk.ktap = 9u * cin;
         Wk.cout = L.cout;
-        Wk.bias = 1;
-        int s = launch_wgrad(Wk, st);
+        int s = launch_wgrad(Wk, plan[l], st);
         if (s != GK_OK) return s;
         if (S.ga == kNone) continue;
         ConvK K{};
@@ -1840,21 +2042,24 @@ int backward(gk_unet& n, const float* target, uint32_t nimg, uint32_t h, uint32_
         K.bias = 0;
         K.out = n.t[S.ga].ptr;
         K.out2 = S.gb == kNone ? nullptr : n.t[S.gb].ptr;
+        if (S.post == 0 && l > 0) K.mask = n.t[S.a].ptr;  // the input is the layer below's output
         s = launch_conv(K, nimg, st);
         if (s != GK_OK) return s;
         if (S.post == 1) {  // gradient of the upsampled input -> low resolution
             const uint32_t c = L.cin_a;
             const size_t cnt = size_t(nimg) * (lh / 2) * (lw / 2) * (c / 8);
-            k_upsum<<<nblk(cnt), 256, 0, st>>>(n.t[S.ga].ptr, n.t[S.post_dst].ptr, nimg, lh, lw, c);
+            k_upsum<<<nblk(cnt), 256, 0, st>>>(n.t[S.ga].ptr, n.t[S.a].ptr, n.t[S.post_dst].ptr, nimg, lh, lw, c);
             GK_HIP(hipGetLastError());
         } else if (S.post == 2) {  // gradient of the pooled input -> the skip tensor above
             const uint32_t c = L.cin_a;
             const uint32_t uh = lh * 2, uw = lw * 2;
             const size_t cnt = size_t(nimg) * lh * lw * (c / 8);
-            k_pool_bwd<<<nblk(cnt), 256, 0, st>>>(n.t[S.ga].ptr, n.t[S.post_dst].ptr, nimg, uh, uw, c);
+            k_pool_bwd<<<nblk(cnt), 256, 0, st>>>(n.t[S.ga].ptr, n.t[kSpec[l - 1].out].ptr, n.t[S.post_dst].ptr, nimg, uh, uw, c);
             GK_HIP(hipGetLastError());
         }
     }
+    k_wgrad_sum<<<uint32_t(n.nparam / 64u), 256, 0, st>>>(sum, grad);
+    GK_HIP(hipGetLastError());
     return GK_OK;
 }
 

@@ -101,6 +101,37 @@ def test_gradient_matches_oracle():
     assert np.all(g[pad] == 0)
 
 
+# widths that are no multiple of a 32-pixel tile row at any level, heights that end inside a
+# tile, a single pixel at the coarsest level, and channel counts that take every split of the
+# weight gradient's waves (1 to 8 input groups, 1 to 3 output tiles, odd and even segments)
+@pytest.mark.parametrize("base,n,h,w", [(32, 1, 16, 16), (32, 2, 48, 80), (8, 3, 64, 32), (16, 1, 16, 112),
+                                        (40, 1, 32, 48), (64, 1, 32, 48)])
+def test_gradient_shapes_match_oracle(base, n, h, w):
+    """As test_gradient_matches_oracle (same bounds: bf16 roundings that the summation order
+    flips), and the same bits on a second call: every sum has a fixed order."""
+    import torch
+    rng = np.random.default_rng(base + h)
+    f = features(rng, n, h, w)
+    t = rng.gamma(1.0, 1.0, (n, h, w, 3)).astype(np.float32)
+    with gk.Context(16, 16) as ctx:
+        net = gk.UNet(ctx, base, seed=3)
+        p = net.get_params()
+        d_in, d_t = torch.from_numpy(f).cuda(), torch.from_numpy(t).cuda()
+        d_g = torch.full((2, net.num_params()), float("nan"), device="cuda")
+        loss = [net.grad(d_in.data_ptr(), d_t.data_ptr(), n, h, w, d_g[k].data_ptr()) for k in (0, 1)]
+        g = d_g.cpu().numpy()
+    assert np.array_equal(g[0], g[1])
+    lo, go = U.loss_grad(p, f, t, base, bf16_mode=True)
+    assert loss[0] == pytest.approx(lo, rel=2e-3)
+    for i, L in enumerate(U.layers(base)):
+        sl = slice(L["offset"], L["offset"] + L["cout"] * L["kpad"])
+        a, b = g[0][sl], go[sl]
+        cos = float(a @ b / (np.linalg.norm(a) * np.linalg.norm(b)))
+        assert rel(a, b) < 3e-2 and cos > 0.999, (i, rel(a, b), cos)
+        M, cin = a.reshape(L["cout"], L["kpad"]), L["cin_a"] + L["cin_b"]
+        assert np.all(M[:, 9 * cin + 1:] == 0)  # padding columns
+
+
 def test_adam_step_and_save_load():
     import torch
     rng = np.random.default_rng(2)
