@@ -12,19 +12,32 @@
 // values it multiplies (f/p with p detached). For a path whose contributions are C_j
 // (emission found at vertex j, or NEE at vertex j) this gives
 //     dC/dtheta = sum_k d log f_k / dtheta * (sum_{j > k} C_j) + sum_j dC_nee_j / dtheta
-// where f_k is the lobe sampled at vertex k. The adjoint replays each path from its seed
-// twice: pass 1 computes the path's total radiance Ltot, pass 2 accumulates the prefix P
-// and uses Ltot - P as the suffix radiance at every vertex (path-replay backpropagation,
-// Vicini, Speierer & Jakob 2021). Nothing is stored per vertex.
+// where f_k is the lobe sampled at vertex k. The adjoint traces each path again from its
+// seed, keeps 36 bytes per scattering vertex (material and lobe, the radiance P found before
+// it, what the lobe's derivative needs) and, once the path has ended and its total radiance
+// Ltot is known, visits them with Ltot - P, the suffix radiance of each. (Replaying the path
+// a second time instead, as path-replay backpropagation does to store nothing, costs a second
+// traversal of the scene.)
 //
 // Parameters per material (5 floats): albedo r, g, b, roughness (fuzziness), metallic.
 // Gradient contributions are summed per work-group in LDS and the per-group partials are
 // added in a fixed order by a second kernel.
+//
+// A wave traces the 8 x 8 pixels of a tile, one sample of each; the waves of a work-group
+// take different samples of the same tile (up to 4) or different tiles.
+//
+// Bound: the traversal (gk_single.hpp), at 3 or 4 waves per SIMD. 512 x 512, 4 spp, 4 bounces,
+// 740 triangles: primal 2.67 ms and adjoint 5.44 ms with one thread per pixel in rows, leaves
+// tested as met, the stack in scratch and every path replayed twice; 2.02 and 2.12 ms with
+// tiles, a wave per sample (the last of 1.3 rounds of resident waves no longer runs four
+// samples) and recorded vertices; 1.04 and 1.25 ms with the traversal of gk_single.hpp.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 
 #include "gk_ptmis.hpp"
+#include "gk_single.hpp"
 
 namespace gk {
 
@@ -36,7 +49,28 @@ struct DiffK {
     float mvi[16], pi[16];
     float sky[4], sky_rot;
     uint32_t W, H, frame0, seed, spp, bounces, has_sky;
+    uint32_t tiles_x, tiles;  // 8 x 8 pixel tiles, the last ones of a row or column partly outside
+    uint32_t streams;         // waves of a work-group on the same tile (1, 2 or 4)
 };
+
+// One scattering vertex of a path under differentiation, in planes of one entry per thread.
+struct PathRec {
+    float4* a;       // material | spec << 31 (bits), radiance found before the vertex
+    float4* b;       // specular lobe: 1 - x5, Fresnel F
+    float* c;        // specular lobe: d log K / d roughness
+    uint32_t plane;  // entries of a plane
+};
+
+// the pixel of this thread in its work-group's it-th tile group, or false outside the image
+__device__ inline bool tile_pixel(const DiffK& K, uint32_t group, uint32_t& x, uint32_t& y) {
+    const uint32_t wv = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+    const uint32_t tile = group * (4u / K.streams) + wv / K.streams;
+    if (tile >= K.tiles) return false;
+    const uint32_t ty = tile / K.tiles_x, tx = tile - ty * K.tiles_x;
+    x = tx * 8u + (lane & 7u);
+    y = ty * 8u + (lane >> 3);
+    return x < K.W && y < K.H;
+}
 
 // camera ray through the image position (fx, fy) in pixels
 __device__ inline void camera_ray(const DiffK& K, float fx, float fy, f3& O, f3& D) {
@@ -94,9 +128,11 @@ __device__ inline SpecParts spec_parts(const Bsdf& b, const gk_material& m, f3 w
 
 __device__ inline bool metal_live(const gk_material& m) { return m.material_model == GK_MATERIAL_MIXTURE; }
 
-template <bool ADJ>
-__device__ inline f3 dpath(const DScene& s, const DiffK& K, uint32_t x, uint32_t y, rng4& seed, f3 dL, f3 Ltot,
-                           float* g /* LDS, 5 per material */) {
+// The path of one sample: its radiance. ADJ: also adds the next-event terms of dL * dC to g
+// and records the scattering vertices (rec, entry gtid of each plane, nrec of them).
+template <bool ADJ, bool TWO>
+__device__ inline f3 dpath(const DScene& s, const DiffK& K, uint32_t x, uint32_t y, rng4& seed, SingleStack stack, f3 dL,
+                           float* g /* LDS, 5 per material */, const PathRec& rec, uint32_t gtid, uint32_t& nrec) {
     f3 O, D;
     float jx, jy;  // sub-pixel position of this sample
     rnd2(seed, jx, jy);
@@ -108,7 +144,7 @@ __device__ inline f3 dpath(const DScene& s, const DiffK& K, uint32_t x, uint32_t
     auto add = [&](f3 C) { Lsum = Lsum + C; };
     for (uint32_t depth = 0;; ++depth) {
         SHit h;
-        if (!trace_closest_single(s, O, D, 0.f, 1e30f, h)) {
+        if (!trace_single<false, TWO>(s, O, D, 0.f, 1e30f, h, stack)) {
             if (K.has_sky) {
                 const float4 sky = sky_radiance(s, K.sky, K.sky_rot, D);
                 add(T * f3{sky.x, sky.y, sky.z});
@@ -193,7 +229,8 @@ __device__ inline f3 dpath(const DScene& s, const DiffK& K, uint32_t x, uint32_t
             const float psel = s.light_cdf[li + 1] - s.light_cdf[li];  // 0: a light switched off
             if (cosl > 0.f && wil.z > 0.f && dot(Ng, wl) > 0.f && psel > 0.f) {
                 const float pl = psel * d2 / (cosl * L.p0.w);
-                if (!occluded_single(s, Po, wl, 0.f, dist * (1.f - 1e-4f) - off)) {
+                SHit unused;
+                if (!trace_single<true, TWO>(s, Po, wl, 0.f, dist * (1.f - 1e-4f) - off, unused, stack)) {
                     f3 fd, fs;
                     float pdd, pds;
                     bsdf_eval(b, wo, wil, fd, fs, pdd, pds);
@@ -250,28 +287,12 @@ __device__ inline f3 dpath(const DScene& s, const DiffK& K, uint32_t x, uint32_t
         const f3 f = f3{spec ? +fs.x : +fd.x, spec ? +fs.y : +fd.y, spec ? +fs.z : +fd.z};
         if (!(pdf > 0.f)) break;
         if (ADJ) {
-            // d log f_lobe / d theta times the suffix radiance Ltot - P
-            const f3 S = (Ltot - Lsum) * dL;
-            float* gm = g + 5 * mi;
+            const size_t e = size_t(nrec++) * rec.plane + gtid;
+            rec.a[e] = make_float4(__uint_as_float(mi | (spec ? 0x80000000u : 0u)), Lsum.x, Lsum.y, Lsum.z);
             if (spec) {
                 const SpecParts sp = spec_parts(b, mat, wo, wi);
-                const float k1 = 1.f - sp.x5;
-                if (sp.F.x > 0.f) atomicAdd(&gm[0], S.x * b.metal * k1 / sp.F.x);
-                if (sp.F.y > 0.f) atomicAdd(&gm[1], S.y * b.metal * k1 / sp.F.y);
-                if (sp.F.z > 0.f) atomicAdd(&gm[2], S.z * b.metal * k1 / sp.F.z);
-                atomicAdd(&gm[3], (S.x + S.y + S.z) * sp.dlogK_dr);
-                if (metal_live(mat)) {
-                    float dm = 0.f;
-                    if (sp.F.x > 0.f) dm += S.x * (b.albedo.x - 0.04f) * k1 / sp.F.x;
-                    if (sp.F.y > 0.f) dm += S.y * (b.albedo.y - 0.04f) * k1 / sp.F.y;
-                    if (sp.F.z > 0.f) dm += S.z * (b.albedo.z - 0.04f) * k1 / sp.F.z;
-                    atomicAdd(&gm[4], dm);
-                }
-            } else {
-                if (b.albedo.x > 0.f) atomicAdd(&gm[0], S.x / b.albedo.x);
-                if (b.albedo.y > 0.f) atomicAdd(&gm[1], S.y / b.albedo.y);
-                if (b.albedo.z > 0.f) atomicAdd(&gm[2], S.z / b.albedo.z);
-                if (metal_live(mat) && b.metal < 1.f) atomicAdd(&gm[4], -(S.x + S.y + S.z) / (1.f - b.metal));
+                rec.b[e] = make_float4(1.f - sp.x5, sp.F.x, sp.F.y, sp.F.z);
+                rec.c[e] = sp.dlogK_dr;
             }
         }
         T = T * f * (wi.z / pdf);
@@ -284,37 +305,95 @@ __device__ inline f3 dpath(const DScene& s, const DiffK& K, uint32_t x, uint32_t
     return Lsum;
 }
 
-__global__ __launch_bounds__(256) void k_diff_primal(DScene s, DiffK K, float4* __restrict__ img) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= K.W * K.H) return;
-    const uint32_t x = i % K.W, y = i / K.W;
-    f3 acc = f3{0.f, 0.f, 0.f};
-    for (uint32_t smp = 0; smp < K.spp; ++smp) {
-        rng4 seed{x, y, K.frame0 + smp, K.seed};
-        acc = acc + dpath<false>(s, K, x, y, seed, f3{0, 0, 0}, f3{0, 0, 0}, nullptr);
+// d log f_lobe / d theta times the suffix radiance Ltot - P of a path's recorded vertices
+__device__ inline void scatter_gradients(const DScene& s, const PathRec& rec, uint32_t gtid, uint32_t nrec, f3 Ltot,
+                                         f3 dL, float* g) {
+    for (uint32_t k = 0; k < nrec; ++k) {
+        const size_t e = size_t(k) * rec.plane + gtid;
+        const float4 a = rec.a[e];
+        const uint32_t mi = __float_as_uint(a.x) & 0x7fffffffu;
+        const gk_material& mat = s.mats[mi];
+        const Bsdf b = bsdf_of(mat);
+        const f3 S = (Ltot - f3{a.y, a.z, a.w}) * dL;
+        float* gm = g + 5 * mi;
+        if (__float_as_uint(a.x) & 0x80000000u) {
+            const float4 q = rec.b[e];
+            const float k1 = q.x;
+            const f3 F = f3{q.y, q.z, q.w};
+            if (F.x > 0.f) atomicAdd(&gm[0], S.x * b.metal * k1 / F.x);
+            if (F.y > 0.f) atomicAdd(&gm[1], S.y * b.metal * k1 / F.y);
+            if (F.z > 0.f) atomicAdd(&gm[2], S.z * b.metal * k1 / F.z);
+            atomicAdd(&gm[3], (S.x + S.y + S.z) * rec.c[e]);
+            if (metal_live(mat)) {
+                float dm = 0.f;
+                if (F.x > 0.f) dm += S.x * (b.albedo.x - 0.04f) * k1 / F.x;
+                if (F.y > 0.f) dm += S.y * (b.albedo.y - 0.04f) * k1 / F.y;
+                if (F.z > 0.f) dm += S.z * (b.albedo.z - 0.04f) * k1 / F.z;
+                atomicAdd(&gm[4], dm);
+            }
+        } else {
+            if (b.albedo.x > 0.f) atomicAdd(&gm[0], S.x / b.albedo.x);
+            if (b.albedo.y > 0.f) atomicAdd(&gm[1], S.y / b.albedo.y);
+            if (b.albedo.z > 0.f) atomicAdd(&gm[2], S.z / b.albedo.z);
+            if (metal_live(mat) && b.metal < 1.f) atomicAdd(&gm[4], -(S.x + S.y + S.z) / (1.f - b.metal));
+        }
     }
-    const float inv = 1.f / float(K.spp);
-    img[i] = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, 1.f);
 }
 
-// grad partials: one row of 5*nmat floats per work-group
-__global__ __launch_bounds__(256) void k_diff_adjoint(DScene s, DiffK K, const float4* __restrict__ dimg,
-                                                      float* __restrict__ partial, uint32_t nparam) {
+// Four waves per SIMD in single-level scenes (126 registers; at 129, three waves, the primal
+// takes 1.21 ms against 1.04 and the adjoint 1.33 against 1.25), three in two-level ones, whose
+// instance handling would spill.
+template <bool TWO>
+__global__ __launch_bounds__(256, TWO ? 3 : 4) void k_diff_primal(DScene s, DiffK K, float4* __restrict__ img) {
+    __shared__ uint32_t stacks[kSingleLds][256];
+    float (*part)[256] = reinterpret_cast<float (*)[256]>(&stacks[0][0]);  // after the paths
+    uint32_t x, y, nrec = 0;
+    const bool in = tile_pixel(K, blockIdx.x, x, y);
+    const uint32_t stream = (threadIdx.x >> 6) % K.streams;
+    f3 acc = f3{0.f, 0.f, 0.f};
+    if (in)
+        for (uint32_t smp = stream; smp < K.spp; smp += K.streams) {
+            rng4 seed{x, y, K.frame0 + smp, K.seed};
+            acc = acc + dpath<false, TWO>(s, K, x, y, seed, (SingleStack)&stacks[0][threadIdx.x], f3{0, 0, 0}, nullptr, PathRec{}, 0u,
+                                           nrec);
+        }
+    __syncthreads();
+    part[0][threadIdx.x] = acc.x;
+    part[1][threadIdx.x] = acc.y;
+    part[2][threadIdx.x] = acc.z;
+    __syncthreads();
+    if (!in || stream != 0u) return;
+    for (uint32_t k = 1; k < K.streams; ++k) {
+        const uint32_t t = threadIdx.x + 64u * k;
+        acc = acc + f3{part[0][t], part[1][t], part[2][t]};
+    }
+    const float inv = 1.f / float(K.spp);
+    img[size_t(y) * K.W + x] = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, 1.f);
+}
+
+// grad partials: one row of 5*nmat floats per work-group; groups: tile groups of the image,
+// which the work-groups of the launch take in turn
+template <bool TWO>
+__global__ __launch_bounds__(256, TWO ? 3 : 4) void k_diff_adjoint(DScene s, DiffK K, const float4* __restrict__ dimg, PathRec rec,
+                                                      float* __restrict__ partial, uint32_t nparam, uint32_t groups) {
     extern __shared__ float g[];
+    __shared__ uint32_t stacks[kSingleLds][256];
     for (uint32_t k = threadIdx.x; k < nparam; k += blockDim.x) g[k] = 0.f;
     __syncthreads();
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < K.W * K.H) {
-        const uint32_t x = i % K.W, y = i / K.W;
+    const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t stream = (threadIdx.x >> 6) % K.streams;
+    for (uint32_t group = blockIdx.x; group < groups; group += gridDim.x) {
+        uint32_t x, y;
+        if (!tile_pixel(K, group, x, y)) continue;
         const float inv = 1.f / float(K.spp);
-        const float4 dl4 = dimg[i];
+        const float4 dl4 = dimg[size_t(y) * K.W + x];
         const f3 dL = f3{dl4.x * inv, dl4.y * inv, dl4.z * inv};  // image = mean over samples
         if (dL.x != 0.f || dL.y != 0.f || dL.z != 0.f) {
-            for (uint32_t smp = 0; smp < K.spp; ++smp) {
+            for (uint32_t smp = stream; smp < K.spp; smp += K.streams) {
                 rng4 seed{x, y, K.frame0 + smp, K.seed};
-                const f3 Ltot = dpath<false>(s, K, x, y, seed, f3{0, 0, 0}, f3{0, 0, 0}, nullptr);
-                rng4 seed2{x, y, K.frame0 + smp, K.seed};
-                dpath<true>(s, K, x, y, seed2, dL, Ltot, g);
+                uint32_t nrec = 0;
+                const f3 Ltot = dpath<true, TWO>(s, K, x, y, seed, (SingleStack)&stacks[0][threadIdx.x], dL, g, rec, gtid, nrec);
+                scatter_gradients(s, rec, gtid, nrec, Ltot, dL, g);
             }
         }
     }
@@ -323,12 +402,20 @@ __global__ __launch_bounds__(256) void k_diff_adjoint(DScene s, DiffK K, const f
     for (uint32_t k = threadIdx.x; k < nparam; k += blockDim.x) row[k] = g[k];
 }
 
-__global__ void k_reduce_partials(const float* __restrict__ partial, uint32_t rows, uint32_t nparam,
+// 32 parameters per work-group, 8 threads of interleaved rows each, added in a fixed order
+// (1024 rows of 1285: 250 us with one thread per parameter over all rows, 40 us now)
+__global__ __launch_bounds__(256) void k_reduce_partials(const float* __restrict__ partial, uint32_t rows, uint32_t nparam,
                                   float* __restrict__ out) {
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= nparam) return;
+    __shared__ double red[8][32];
+    const uint32_t c = threadIdx.x & 31u, r0 = threadIdx.x >> 5;
+    const uint32_t k = blockIdx.x * 32u + c;
     double acc = 0.0;
-    for (uint32_t r = 0; r < rows; ++r) acc += double(partial[size_t(r) * nparam + k]);
+    if (k < nparam)
+        for (uint32_t r = r0; r < rows; r += 8u) acc += double(partial[size_t(r) * nparam + k]);
+    red[r0][c] = acc;
+    __syncthreads();
+    if (r0 != 0u || k >= nparam) return;
+    for (int q = 1; q < 8; ++q) acc += red[q][c];
     out[k] = float(acc);
 }
 
@@ -345,7 +432,17 @@ DiffK make_diffk(const Ctx& c) {
     K.spp = c.params.samples > 0 ? c.params.samples : 1;
     K.bounces = c.params.bounces;
     K.has_sky = c.params.has_sky;
+    K.tiles_x = (K.W + 7u) / 8u;
+    K.tiles = K.tiles_x * ((K.H + 7u) / 8u);
+    K.streams = K.spp >= 4u ? 4u : (K.spp >= 2u ? 2u : 1u);
     return K;
+}
+
+constexpr size_t kRecBytes = size_t(96) << 20;
+
+uint32_t tile_groups(const DiffK& K) {
+    const uint32_t per = 4u / K.streams;
+    return (K.tiles + per - 1u) / per;
 }
 
 }  // namespace
@@ -367,9 +464,9 @@ int gk_render_radiance(gk_ctx* ctx, float* d_image) {
         const int st = refit_tlas(c);
         if (st != GK_OK) return st;
     }
-    const uint32_t n = c.width * c.height;
-    k_diff_primal<<<(n + 255) / 256, 256, 0, c.stream>>>(make_dscene(c), make_diffk(c),
-                                                          reinterpret_cast<float4*>(d_image));
+    const DiffK K = make_diffk(c);
+    auto* kern = c.blas_only ? k_diff_primal<false> : k_diff_primal<true>;
+    kern<<<tile_groups(K), 256, 0, c.stream>>>(make_dscene(c), K, reinterpret_cast<float4*>(d_image));
     GK_HIP(hipGetLastError());
     return GK_OK;
 }
@@ -387,14 +484,31 @@ int gk_adjoint(gk_ctx* ctx, const float* d_dl_dimage, float* d_grad) {
         const int st = refit_tlas(c);
         if (st != GK_OK) return st;
     }
-    const uint32_t n = c.width * c.height;
-    const uint32_t blocks = (n + 255) / 256;
+    const DiffK K = make_diffk(c);
+    const uint32_t groups = tile_groups(K);
+    // work-groups: as many as are resident (4 or 3 per CU), since each writes a row of
+    // gradients; fewer where the records of so many paths would pass kRecBytes (more than 10
+    // bounces) or the image has fewer tile groups
+    const uint32_t verts = std::max(1u, K.bounces);
+    const uint32_t resident = c.blas_only ? 1024u : 768u;
+    const uint32_t blocks = std::min(groups, std::min(resident, uint32_t(kRecBytes / (size_t(256) * verts * 36u))));
+    const size_t plane = size_t(blocks) * 256u;
     if (c.grad_partial.count < size_t(blocks) * nparam) GK_HIP(c.grad_partial.resize(size_t(blocks) * nparam));
-    k_diff_adjoint<<<blocks, 256, nparam * 4, c.stream>>>(make_dscene(c), make_diffk(c),
-                                                          reinterpret_cast<const float4*>(d_dl_dimage),
-                                                          c.grad_partial.ptr, nparam);
+    if (c.path_rec.count < plane * verts * 9u) GK_HIP(c.path_rec.resize(plane * verts * 9u));
+    PathRec rec;
+    rec.a = reinterpret_cast<float4*>(c.path_rec.ptr);
+    rec.b = rec.a + plane * verts;
+    rec.c = reinterpret_cast<float*>(rec.b + plane * verts);
+    rec.plane = uint32_t(plane);
+    auto* kern = c.blas_only ? k_diff_adjoint<false> : k_diff_adjoint<true>;
+    // gradients (dynamic) and traversal stacks (static) above the default 64 KB of LDS
+    if (nparam * 4u + kSingleLds * 1024u > 65536u)
+        GK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   int(nparam * 4u)));
+    kern<<<blocks, 256, nparam * 4, c.stream>>>(make_dscene(c), K, reinterpret_cast<const float4*>(d_dl_dimage), rec,
+                                                c.grad_partial.ptr, nparam, groups);
     GK_HIP(hipGetLastError());
-    k_reduce_partials<<<(nparam + 255) / 256, 256, 0, c.stream>>>(c.grad_partial.ptr, blocks, nparam, d_grad);
+    k_reduce_partials<<<(nparam + 31) / 32, 256, 0, c.stream>>>(c.grad_partial.ptr, blocks, nparam, d_grad);
     GK_HIP(hipGetLastError());
     return GK_OK;
 }

@@ -230,3 +230,67 @@ def test_descent_recovers_perturbed_parameters_from_an_independent_target():
     print(f"albedo error over {int(seen.sum())} materials: {err0:.4f} -> {err1:.4f}; "
           f"loss {np.mean(losses[:5]):.3e} -> {np.mean(losses[-5:]):.3e}")
     assert err1 < 0.5 * err0, (err0, err1)
+
+
+# tiles cut by the image's edge, one to five samples (one, two or four waves on a tile), a
+# single bounce, more bounces than records of all resident paths fit in the record buffer, and
+# a scene of two instances (the two-level traversal)
+@pytest.mark.parametrize("W,H,spp,bounces,instances", [(8, 8, 1, 1, 1), (13, 29, 2, 4, 1), (50, 41, 3, 4, 2),
+                                                       (33, 16, 5, 12, 1), (64, 64, 4, 64, 2)])
+def test_shapes_match_oracle_and_single_samples(W, H, spp, bounces, instances):
+    """The image equals the oracle's render; the image and the gradient of spp samples are the
+    means of those of the samples rendered one at a time (32-bit sums in another order)."""
+    import torch
+    from gknextengine_amd import diff
+    scene, nmat, p = setup(W, H, spp, bounces)
+    if instances == 2:
+        w = np.eye(4, dtype=np.float32)
+        w[0, 3] = 1.5
+        scene.add_instance(0, world=w)
+    base = list(scene.materials)
+    dL = torch.from_numpy(np.random.default_rng(W).normal(size=(H, W, 3)).astype(np.float32)).cuda()
+    ref = po.OracleScene(scene).diff_render(p, W, H, spp=spp, frame0=p.total_frames)
+
+    def both(q):
+        x = diff.params_of(base).cuda().requires_grad_(True)
+        img = diff.render(x, ctx, base, q, decorrelate=False)
+        (img * dL).sum().backward()
+        return img.detach(), x.grad
+
+    with gk.Context(W, H) as ctx:
+        ctx.upload(scene)
+        img, g = both(p)
+        parts = []
+        for k in range(spp):
+            q = gk.FrameParams.from_buffer_copy(p)
+            q.samples, q.total_frames = 1, p.total_frames + k
+            parts.append(both(q))
+    close = np.all(np.abs(img.cpu().numpy() - ref) <= 1e-3 * (1 + np.abs(ref)), axis=2)
+    assert close.mean() > 0.95, close.mean()
+    mean_img = sum(a for a, _ in parts) / spp
+    mean_g = sum(b for _, b in parts) / spp
+    assert torch.allclose(img, mean_img, rtol=1e-5, atol=1e-6)
+    assert torch.allclose(g, mean_g, rtol=1e-4, atol=2e-6 * float(mean_g.abs().max())), (g - mean_g).abs().max()
+
+
+@pytest.mark.parametrize("count", [600, 2458, 3276])
+def test_material_count_up_to_the_limit(count):
+    """Materials no triangle uses get a zero gradient and leave the others' unchanged, up to the
+    3276 whose sums fit the work-groups (2458 and more pass 64 KB of LDS with the stacks)."""
+    import torch
+    from gknextengine_amd import diff
+    W = H = 24
+    scene, nmat, p = setup(W, H, spp=2)
+    base = list(scene.materials)
+    dL = torch.from_numpy(np.random.default_rng(8).normal(size=(H, W, 3)).astype(np.float32)).cuda()
+    grads = []
+    for mats in (base, base + [copy.deepcopy(base[0]) for _ in range(count - len(base))]):
+        scene.materials = mats
+        with gk.Context(W, H) as ctx:
+            ctx.upload(scene)
+            x = diff.params_of(mats).cuda().requires_grad_(True)
+            (diff.render(x, ctx, mats, p, decorrelate=False) * dL).sum().backward()
+            grads.append(x.grad.clone())
+    n = len(base)
+    assert torch.all(grads[1][n:] == 0)
+    assert torch.allclose(grads[1][:n], grads[0], rtol=1e-4, atol=2e-6 * float(grads[0].abs().max()))
