@@ -308,7 +308,7 @@ int launch_trace(Ctx& c, const float4* ray_o, const float4* ray_d, const uint32_
 // a closest-hit queue (o, d -> hit, hit_inst) and an occlusion queue (so, sd -> shit) in one launch
 int launch_trace_pair(Ctx& c, const float4* o, const float4* d, const uint32_t* count_dev, uint32_t max_count,
                       float4* hit, uint32_t* hit_inst, const float4* so, const float4* sd,
-                      const uint32_t* scount_dev, uint32_t smax_count, float4* shit, int slot = 0);
+                      const uint32_t* scount_dev, uint32_t smax_count, float4* shit, uint32_t* clear, int slot = 0);
 int launch_trace_user(Ctx& c, const gk_ray* rays, uint32_t n, gk_hit* hits, uint32_t* inst, uint32_t flags);
 // the ray counter a trace launch in `slot` starts from (allocates the slot's spill area); a
 // caller whose kernel zeroed it sets Ctx::trace_counter_zeroed[slot], and the next launch in

@@ -569,7 +569,7 @@ int probes_bake(Ctx& c, uint32_t first, uint32_t count) {
         if (K.nany)
             st = launch_trace_pair(c, W.ro.ptr, W.rd.ptr, W.counters.ptr + 1, n * kProbeRays, W.hit.ptr,
                                    W.hit_inst.ptr, W.so.ptr, W.sd.ptr, W.counters.ptr + 2, n * 6u * K.nany,
-                                   W.shit.ptr, h);
+                                   W.shit.ptr, nullptr, h);
         else
             st = launch_trace(c, W.ro.ptr, W.rd.ptr, W.counters.ptr + 1, n * kProbeRays, W.hit.ptr, W.hit_inst.ptr,
                               false, nullptr, h);

@@ -454,6 +454,7 @@ __global__ __launch_bounds__(kBlock) void k_trace(
     const uint32_t count = c0 + c1;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         if (j0.clear) *j0.clear = 0u;
+        if (MODE == 2 && j1.clear) *j1.clear = 0u;
         atomicAdd(&ray_stats[MODE == 1 ? 1 : 0], (unsigned long long)c0);
         if (MODE == 2) atomicAdd(&ray_stats[1], (unsigned long long)c1);
     }
@@ -787,12 +788,13 @@ int launch_trace(Ctx& c, const float4* ray_o, const float4* ray_d, const uint32_
     return launch_jobs(c, any_hit ? 1 : 0, j0, TraceJob{}, slot);
 }
 
-// A closest-hit queue and an occlusion queue in one launch.
+// A closest-hit queue and an occlusion queue in one launch. clear (device, may be null): two
+// words the launch zeroes, the sizes of the queues the shading after it appends to.
 int launch_trace_pair(Ctx& c, const float4* o, const float4* d, const uint32_t* count_dev, uint32_t max_count,
                       float4* hit, uint32_t* hit_inst, const float4* so, const float4* sd,
-                      const uint32_t* scount_dev, uint32_t smax_count, float4* shit, int slot) {
-    const TraceJob j0{o, d, count_dev, max_count, hit, hit_inst, nullptr};
-    const TraceJob j1{so, sd, scount_dev, smax_count, shit, nullptr, nullptr};
+                      const uint32_t* scount_dev, uint32_t smax_count, float4* shit, uint32_t* clear, int slot) {
+    const TraceJob j0{o, d, count_dev, max_count, hit, hit_inst, clear};
+    const TraceJob j1{so, sd, scount_dev, smax_count, shit, nullptr, clear ? clear + 1 : nullptr};
     return launch_jobs(c, 2, j0, j1, slot);
 }
 

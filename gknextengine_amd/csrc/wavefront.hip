@@ -112,10 +112,11 @@ struct PathState {
     uint4* misc;    // x pixel, y flags, z counters, w material of the current vertex
     float4* pos;    // current vertex position (w: primary material bits for REF_V2)
     float4* nrm;    // current vertex normal
-    float4* dir;    // current incoming direction
+    float4* dir;    // current incoming direction (w: slot of a pending sun ray)
     float4* ppos;   // REF_V2 primary vertex (pulled back), w = primary material bits
     float4* pnrm;   // REF_V2 primary normal
     float4* palb;   // REF_V2 primary albedo (FetchGBufferV2: textured)
+    uint4* rng2;    // REF_V2: random state after the draws of a pending sun ray
 };
 
 // Path p -> pixel. Tiled frames walk 8x8 tiles, 64 paths each, in parts: part h of the path
@@ -437,7 +438,9 @@ __global__ void k_vis_primary(DScene s, FrameK K, Queues Q, const uint32_t* __re
 
 // ================================================================ REF_V2
 // flags (misc.y): bit0 chanceReflect of the pending GetRayColor, bit1 BackFace,
-// bit2 origin material is dielectric, bit3 hitReflect (first call), bit4 hitMetal (first call)
+// bit2 origin material is dielectric, bit3 hitReflect (first call), bit4 hitMetal (first call),
+// bit5 the vertex's sun ray is pending, bit6 the pixel's last one (DirectIlluminate) is, bit7
+// with bit5: the sample ends there also when the sun is hidden
 // counters (misc.z): bits 0-7 bounce b of the pending call, 8-19 sample, 20-31 sample count - 1
 // (gk_frame allows 1024 samples, x4 on moving pixels: 4096 samples, indices 0..4095)
 
@@ -478,45 +481,32 @@ __device__ inline void ref_begin(const DScene& s, const FrameK& K, const Queues&
     (void)Q;
 }
 
-// end of a sample (Shading.slang:1159-1171); restarts the next sample or finalizes
-__device__ inline void ref_end_sample(const DScene& s, const FrameK& K, const Targets& T, const PathState& S,
-                                      uint32_t p, uint32_t px, float4 color, uint32_t& flags, uint32_t& counters,
-                                      rng4& seed, bool& emit, float4& ro, float4& rd) {
-    const float4 pp = S.ppos[p];
-    const uint32_t pmat = __float_as_uint(pp.w);
-    if (flags & 16u) {
-        const float4 pa = S.palb[p];
-        color.x = color.x * pa.x; color.y = color.y * pa.y;
-        color.z = color.z * pa.z; color.w = color.w * pa.w;
-    }
-    float4 acc = (flags & 8u) ? S.ls[p] : S.ld[p];
-    acc.x = acc.x + color.x; acc.y = acc.y + color.y; acc.z = acc.z + color.z; acc.w = acc.w + color.w;
-    if (flags & 8u) S.ls[p] = acc; else S.ld[p] = acc;
-    const uint32_t sample = ((counters >> 8) & 0xfffu) + 1u;
+// a cone sample around the sun (cos of 0.25 degrees), as a ray of the sun queue
+__device__ inline void sun_ray(const FrameK& K, f3 org, rng4& seed, float4& so, float4& sd) {
+    const f3 sun = f3{K.sun_dir[0], K.sun_dir[1], K.sun_dir[2]};
+    const f3 cone = align_with_normal(random_in_cone(seed, 0.99999048072578f), sun);
+    so = make_float4(org.x, org.y, org.z, kEps);
+    sd = make_float4(cone.x, cone.y, cone.z, kMaxTrace);
+}
+
+// an extension queue entry that traces nothing: every box lies behind it
+__device__ inline void null_ray(float4& ro, float4& rd) {
+    ro = make_float4(1e30f, 0.f, 0.f, kEps);
+    rd = make_float4(1.f, 0.f, 0.f, 0.f);
+}
+
+// average and DirectIlluminate (Shading.slang:1175-1183, 888-905) of a path whose samples are
+// done; shadow: 1 when the sun is seen from the primary vertex
+__device__ inline void ref_finish(const FrameK& K, const Targets& T, const PathState& S, uint32_t p, uint32_t px,
+                                  uint32_t counters, float shadow) {
     const uint32_t nsamp = (counters >> 20) + 1u;
-    const f3 ppos = ld3(pp), pnrm = ld3(S.pnrm[p]);
-    if (sample < nsamp) {
-        counters = (counters & 0xfff00000u) | (sample << 8);
-        float e4[4];
-        mul44v(K.mvi, 0.f, 0.f, 0.f, 1.f, e4);
-        const f3 dir = normalize(ppos - f3{e4[0], e4[1], e4[2]});
-        S.thr[p] = make_float4(1.f, 1.f, 1.f, 1.f);
-        ref_begin(s, K, Queues{}, S, p, ppos, pnrm, pmat, dir, seed, flags, 0u, 0, emit, ro, rd);
-        return;
-    }
-    // finalize: average, DirectIlluminate (Shading.slang:1175-1183, 888-905)
+    const f3 pnrm = ld3(S.pnrm[p]);
     float4 fc = S.ld[p], fr = S.ls[p];
     const float ns = float(nsamp);
     fc.x = fc.x / ns; fc.y = fc.y / ns; fc.z = fc.z / ns; fc.w = fc.w / ns;
     fr.x = fr.x / ns; fr.y = fr.y / ns; fr.z = fr.z / ns; fr.w = fr.w / ns;
     const f3 sun = f3{K.sun_dir[0], K.sun_dir[1], K.sun_dir[2]};
     const float d = fmaxf(dot(sun, normalize(pnrm)), 0.0f) * (1.0f / kPi);
-    float shadow = 0.f;
-    if (K.has_sun) {
-        const float cos_cone = 0.99999048072578f;  // cos(0.25 deg)
-        const f3 cone = align_with_normal(random_in_cone(seed, cos_cone), sun);
-        shadow = occluded_single(s, ppos, cone, kEps, kMaxTrace) ? 0.f : 1.f;
-    }
     fc.x = fc.x + K.sun_col[0] * d * shadow; fc.y = fc.y + K.sun_col[1] * d * shadow;
     fc.z = fc.z + K.sun_col[2] * d * shadow; fc.w = fc.w + K.sun_col[3] * d * shadow;
     T.diffuse[px] = to_h4(fc.x, fc.y, fc.z, fc.w);
@@ -530,7 +520,45 @@ __device__ inline void ref_end_sample(const DScene& s, const FrameK& K, const Ta
         q.w += 1.0;
         T.radiance64[px] = q;
     }
+}
+
+// end of a sample (Shading.slang:1159-1171); restarts the next sample or finalizes (SUN: once
+// the sun ray emitted here is answered)
+template <bool SUN>
+__device__ inline void ref_end_sample(const DScene& s, const FrameK& K, const Targets& T, const PathState& S,
+                                      uint32_t p, uint32_t px, float4 color, uint32_t& flags, uint32_t& counters,
+                                      rng4& seed, bool& emit, float4& ro, float4& rd, bool& emit_sun, float4& so,
+                                      float4& sd) {
+    const float4 pp = S.ppos[p];
+    const uint32_t pmat = __float_as_uint(pp.w);
+    if (flags & 16u) {
+        const float4 pa = S.palb[p];
+        color.x = color.x * pa.x; color.y = color.y * pa.y;
+        color.z = color.z * pa.z; color.w = color.w * pa.w;
+    }
+    float4 acc = (flags & 8u) ? S.ls[p] : S.ld[p];
+    acc.x = acc.x + color.x; acc.y = acc.y + color.y; acc.z = acc.z + color.z; acc.w = acc.w + color.w;
+    if (flags & 8u) S.ls[p] = acc; else S.ld[p] = acc;
+    const uint32_t sample = ((counters >> 8) & 0xfffu) + 1u;
+    const uint32_t nsamp = (counters >> 20) + 1u;
+    const f3 ppos = ld3(pp);
     emit = false;
+    if (sample < nsamp) {
+        const f3 pnrm = ld3(S.pnrm[p]);
+        counters = (counters & 0xfff00000u) | (sample << 8);
+        float e4[4];
+        mul44v(K.mvi, 0.f, 0.f, 0.f, 1.f, e4);
+        const f3 dir = normalize(ppos - f3{e4[0], e4[1], e4[2]});
+        S.thr[p] = make_float4(1.f, 1.f, 1.f, 1.f);
+        ref_begin(s, K, Queues{}, S, p, ppos, pnrm, pmat, dir, seed, flags, 0u, 0, emit, ro, rd);
+    } else if (SUN) {
+        sun_ray(K, ppos, seed, so, sd);
+        null_ray(ro, rd);
+        flags |= 64u;
+        emit = emit_sun = true;
+    } else {
+        ref_finish(K, T, S, p, px, counters, 0.f);
+    }
 }
 
 // trace_next: the ray counter of the trace launch that follows, zeroed here
@@ -608,6 +636,18 @@ __global__ __launch_bounds__(256) void k_ref_primary(DScene s, FrameK K, Targets
 
 // GetRayColor after the trace (Shading.slang:1039-1081) and the Render loop body
 // (Shading.slang:1117-1171); cur = queue the hits belong to; trace_next as k_ref_primary.
+// SUN: sun rays (a vertex's, and the one that ends a pixel) go to the occlusion queue of the
+// bounce, traced in one launch with its extension rays; the path's extension entry finds its
+// answer in the next launch (slot in S.dir's w). The vertex goes on as if the sun were hidden,
+// so that a bounce stays one launch: where the sun is then seen, the sample ends with it from
+// the random state kept in S.rng2 and the extension hit is dropped. A path that only waits for
+// its sun ray has an extension entry that traces nothing (null_ray).
+// (Traced inside this kernel by one thread each, with the stack in scratch, the sun rays took
+// most of it: 1080p city with sun, sky and probes 16.7 ms for four frames, 13.5 now, with the
+// probe lookup of gk_probe.hpp. In a queue that delayed their paths by a launch: 14.7 ms, twice
+// the launches, of which the last ten hold a few hundred paths and take as long as their
+// dependent loads, 25 to 80 us each. Four waves per SIMD instead of three spill: 14.0 ms.)
+template <bool SUN>
 __global__ __launch_bounds__(256) void k_ref_shade(DScene s, FrameK K, Targets T, Queues Q, PathState S, int cur,
                                                    uint32_t* __restrict__ trace_next) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -615,114 +655,134 @@ __global__ __launch_bounds__(256) void k_ref_shade(DScene s, FrameK K, Targets T
     const uint32_t n = Q.cnt[2 * cur];
     const int nxt = cur ^ 1;
     const bool live = i < n;
-    bool emit = false;
-    float4 ro{}, rd{};
+    bool emit = false, emit_sun = false;
+    float4 ro{}, rd{}, so{}, sd{};
     uint32_t p = 0;
     if (live) {
         p = Q.path[cur][i];
         uint4 misc = S.misc[p];
         const uint32_t px = misc.x;
         uint32_t flags = misc.y, counters = misc.z, mi = misc.w;
-        const uint4 sr = S.rng[p];
-        rng4 seed{sr.x, sr.y, sr.z, sr.w};
-        float4 color = S.thr[p];
-        const float4 h = Q.hit[i];
-        const uint32_t inst = Q.hit_inst[i];
-        const uint32_t b = counters & 0xffu;
-        const bool chance_reflect = flags & 1u, back = flags & 2u, origin_diel = flags & 4u;
-        bool ret;
-        f3 pos = ld3(S.pos[p]), nrm = ld3(S.nrm[p]);
-        const f3 dir = ld3(S.dir[p]);
-        if (__float_as_uint(h.w) != kMiss) {
-            const f3 O = ld3(Q.o[cur][i]);
-            const uint32_t prim = __float_as_uint(h.w);
-            hit_vertex(s, inst, prim, h.x, h.y, h.z, O, dir, pos, nrm);
-            mi = material_of(s, inst, prim);
-            const gk_material& hm = s.mats[mi];
-            const bool hit_light = hm.material_model == GK_MATERIAL_DIFFUSE_LIGHT;
-            if (hit_light || !chance_reflect) {
-                const float4 ha = mat_albedo(s, hm, hit_uv(s, inst, prim, h.y, h.z));
-                color.x = color.x * ha.x; color.y = color.y * ha.y;
-                color.z = color.z * ha.z; color.w = color.w * ha.w;
-            }
-            if (back && !origin_diel) {
-                color = make_float4(0.5f, 0.5f, 0.5f, 0.f);
-                ret = true;
-            } else {
-                ret = hit_light;
-            }
+        const float4 dir4 = S.dir[p];
+        const bool pending = SUN && (flags & 96u);
+        const bool sun_seen = pending && __float_as_uint(Q.shit[__float_as_uint(dir4.w)].w) == 0u;
+        if (SUN && (flags & 64u)) {
+            ref_finish(K, T, S, p, px, counters, sun_seen ? 1.f : 0.f);
         } else {
-            const float4 sky = K.has_sky ? sky_radiance(s, K.sky, K.sky_rot, dir) : make_float4(0, 0, 0, 0);
-            color.x = color.x * sky.x; color.y = color.y * sky.y; color.z = color.z * sky.z; color.w = color.w * sky.w;
-            ret = true;
-        }
-        const float4 pp = S.ppos[p];
-        const uint32_t pmat = __float_as_uint(pp.w);
-        const bool prim_diel = s.mats[pmat].material_model == GK_MATERIAL_DIELECTRIC;
-        const uint32_t maxb = prim_diel ? K.max_bounces : K.bounces;
-        bool end_sample = false;
-        if (b == 0u) {
-            if (ret || !(1u < maxb)) {
+            const uint4 sr = sun_seen ? S.rng2[p] : S.rng[p];
+            rng4 seed{sr.x, sr.y, sr.z, sr.w};
+            float4 color = S.thr[p];
+            const uint32_t b = counters & 0xffu;
+            f3 pos = ld3(S.pos[p]), nrm = ld3(S.nrm[p]);
+            const f3 dir = ld3(dir4);
+            const float4 pp = S.ppos[p];
+            const uint32_t pmat = __float_as_uint(pp.w);
+            const bool prim_diel = s.mats[pmat].material_model == GK_MATERIAL_DIELECTRIC;
+            const uint32_t maxb = prim_diel ? K.max_bounces : K.bounces;
+            const bool last = flags & 128u;
+            flags &= ~160u;
+            bool end_sample = false, lookup = false;
+            if (sun_seen) {
+                color.x = color.x * K.sun_col[0]; color.y = color.y * K.sun_col[1];
+                color.z = color.z * K.sun_col[2]; color.w = color.w * K.sun_col[3];
                 end_sample = true;
-            } else if (K.fast_gather && !prim_diel) {
-                // ExitAfterFirst (Shading.slang:1118-1124): the probe lookup at the first
-                // bounce's vertex ends the sample
+            } else if (SUN && last) {
+                lookup = true;
+            } else {
+                const float4 h = Q.hit[i];
+                const uint32_t inst = Q.hit_inst[i];
+                const bool chance_reflect = flags & 1u, back = flags & 2u, origin_diel = flags & 4u;
+                bool ret;
+                if (__float_as_uint(h.w) != kMiss) {
+                    const f3 O = ld3(Q.o[cur][i]);
+                    const uint32_t prim = __float_as_uint(h.w);
+                    hit_vertex(s, inst, prim, h.x, h.y, h.z, O, dir, pos, nrm);
+                    mi = material_of(s, inst, prim);
+                    const gk_material& hm = s.mats[mi];
+                    const bool hit_light = hm.material_model == GK_MATERIAL_DIFFUSE_LIGHT;
+                    if (hit_light || !chance_reflect) {
+                        const float4 ha = mat_albedo(s, hm, hit_uv(s, inst, prim, h.y, h.z));
+                        color.x = color.x * ha.x; color.y = color.y * ha.y;
+                        color.z = color.z * ha.z; color.w = color.w * ha.w;
+                    }
+                    if (back && !origin_diel) {
+                        color = make_float4(0.5f, 0.5f, 0.5f, 0.f);
+                        ret = true;
+                    } else {
+                        ret = hit_light;
+                    }
+                } else {
+                    const float4 sky = K.has_sky ? sky_radiance(s, K.sky, K.sky_rot, dir) : make_float4(0, 0, 0, 0);
+                    color.x = color.x * sky.x; color.y = color.y * sky.y; color.z = color.z * sky.z; color.w = color.w * sky.w;
+                    ret = true;
+                }
+                if (b == 0u) {
+                    if (ret || !(1u < maxb)) end_sample = true;
+                    // ExitAfterFirst (Shading.slang:1118-1124): the probe lookup at the first
+                    // bounce's vertex ends the sample
+                    else if (K.fast_gather && !prim_diel) lookup = true;
+                } else if (ret) {
+                    end_sample = true;
+                } else {
+                    if (SUN && rnd1(seed) < 0.5f) {
+                        sun_ray(K, pos + nrm * 0.0f, seed, so, sd);
+                        S.rng2[p] = make_uint4(seed.x, seed.y, seed.z, seed.w);
+                        flags |= 32u;
+                        emit_sun = true;
+                    }
+                    const bool early = !prim_diel && rnd1(seed) < K.exit_prob;
+                    if (b == maxb - 1u || early) {
+                        if (emit_sun) {
+                            flags |= 128u;
+                            null_ray(ro, rd);
+                            emit = true;
+                        } else {
+                            lookup = true;
+                        }
+                    }
+                }
+            }
+            if (lookup) {
+                // RayColor *= interpolateAmbientCubesV2<FullAmbientCubeSampler>(vertex)
                 const float4 pr = probe_lookup<true>(K.probes, pos, nrm);
                 color.x = color.x * pr.x; color.y = color.y * pr.y;
                 color.z = color.z * pr.z; color.w = color.w * pr.w;
                 end_sample = true;
             }
-        } else {
-            if (ret) {
-                end_sample = true;
+            if (end_sample) {
+                ref_end_sample<SUN>(s, K, T, S, p, px, color, flags, counters, seed, emit, ro, rd, emit_sun, so, sd);
+                if (emit) {
+                    // restarted sample: vertex = primary
+                    mi = pmat;
+                    pos = ld3(pp);
+                    nrm = ld3(S.pnrm[p]);
+                    counters = counters & ~0xffu;
+                }
             } else {
-                bool done = false;
-                if (K.has_sun && rnd1(seed) < 0.5f) {
-                    const f3 sun = f3{K.sun_dir[0], K.sun_dir[1], K.sun_dir[2]};
-                    const f3 cone = align_with_normal(random_in_cone(seed, 0.99999048072578f), sun);
-                    if (!occluded_single(s, pos + nrm * 0.0f, cone, kEps, kMaxTrace)) {
-                        color.x = color.x * K.sun_col[0]; color.y = color.y * K.sun_col[1];
-                        color.z = color.z * K.sun_col[2]; color.w = color.w * K.sun_col[3];
-                        done = true;
-                    }
+                S.thr[p] = color;
+                if (!emit) {
+                    const uint32_t nb = b + 1u;
+                    counters = (counters & ~0xffu) | nb;
+                    ref_begin(s, K, Q, S, p, pos, nrm, mi, dir, seed, flags, nb, nxt, emit, ro, rd);
                 }
-                if (!done) {
-                    const bool early = !prim_diel && rnd1(seed) < K.exit_prob;
-                    if (b == maxb - 1u || early) {
-                        // RayColor *= interpolateAmbientCubesV2<FullAmbientCubeSampler>(vertex)
-                        const float4 pr = probe_lookup<true>(K.probes, pos, nrm);
-                        color.x = color.x * pr.x; color.y = color.y * pr.y;
-                        color.z = color.z * pr.z; color.w = color.w * pr.w;
-                        done = true;
-                    }
-                }
-                end_sample = done;
             }
+            S.pos[p] = make_float4(pos.x, pos.y, pos.z, 0.f);
+            S.nrm[p] = make_float4(nrm.x, nrm.y, nrm.z, 0.f);
+            S.misc[p] = make_uint4(px, flags, counters, mi);
+            S.rng[p] = make_uint4(seed.x, seed.y, seed.z, seed.w);
         }
-        if (end_sample) {
-            ref_end_sample(s, K, T, S, p, px, color, flags, counters, seed, emit, ro, rd);
-            if (emit) mi = pmat;
-        } else {
-            const uint32_t nb = b + 1u;
-            counters = (counters & ~0xffu) | nb;
-            S.thr[p] = color;
-            ref_begin(s, K, Q, S, p, pos, nrm, mi, dir, seed, flags, nb, nxt, emit, ro, rd);
-        }
-        if (emit && end_sample) {
-            // restarted sample: vertex = primary
-            pos = ld3(pp);
-            nrm = ld3(S.pnrm[p]);
-            counters = counters & ~0xffu;
-        } else if (!end_sample) {
-            // keep RayColor
-        }
-        if (!end_sample) S.thr[p] = color;
-        S.pos[p] = make_float4(pos.x, pos.y, pos.z, 0.f);
-        S.nrm[p] = make_float4(nrm.x, nrm.y, nrm.z, 0.f);
-        S.misc[p] = make_uint4(px, flags, counters, mi);
-        S.rng[p] = make_uint4(seed.x, seed.y, seed.z, seed.w);
     }
-    const uint32_t slot = block_append(&Q.cnt[2 * nxt], emit);
+    uint32_t slot, ss;
+    if (SUN) {
+        block_append_pair(&Q.cnt[2 * nxt], emit, slot, emit_sun, ss);
+        if (emit_sun) {
+            Q.so[ss] = so;
+            Q.sd[ss] = sd;
+            S.dir[p].w = __uint_as_float(ss);
+        }
+    } else {
+        slot = block_append(&Q.cnt[2 * nxt], emit);
+    }
     if (emit) { Q.o[nxt][slot] = ro; Q.d[nxt][slot] = rd; Q.path[nxt][slot] = p; }
 }
 
@@ -1260,6 +1320,7 @@ int render_frame(Ctx& c) {
     P.thr = w.s_thr.ptr; P.ld = w.s_ld.ptr; P.ls = w.s_ls.ptr; P.rng = w.s_rng.ptr; P.misc = w.s_misc.ptr;
     P.pos = w.s_pos.ptr; P.nrm = w.s_nrm.ptr; P.dir = w.s_dir.ptr; P.ppos = w.s_ppos.ptr; P.pnrm = w.s_pnrm.ptr;
     P.palb = w.s_palb.ptr;
+    P.rng2 = w.q_rng[0].ptr;  // queue state of PT_MIS, free in REF_V2
 
     // previous object ids for reprojection (copy pass, PathTracingRenderer.cpp:160-216)
     k_copy_objid<<<nblk(n), 256, 0, s>>>(T.objid, static_cast<uint32_t*>(c.target_ptr[GK_RT_OBJECTID_1]), n);
@@ -1361,10 +1422,12 @@ int render_frame(Ctx& c) {
             GK_HIP(hipGetLastError());
         }
         cur = 1;
+        const bool sun = K.has_sun != 0u;
         // worst case: every sample uses all bounces (samples * 4 for moving pixels); a sample
-        // traces at least once, also with no bounces
+        // traces at least once, also with no bounces; with a sun the pixel waits once more for
+        // its last sun ray
         const uint32_t maxb = std::max(1u, std::max(K.bounces, K.max_bounces));
-        const uint32_t iters = maxb * K.samples * 4u + 4u;
+        const uint32_t iters = maxb * K.samples * 4u + (sun ? 5u : 4u);
         // A pipeline's loop ends early once the queue it is about to trace is empty: every
         // sample has finished. Reading the counters back costs a synchronisation of the
         // streams, so they are read after the iterations a pixel without motion can take,
@@ -1372,14 +1435,14 @@ int render_frame(Ctx& c) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         GK_HIP(hipStreamIsCapturing(s, &cap));
         if (cap == hipStreamCaptureStatusNone && !c.h_word) GK_HIP(hipHostMalloc(&c.h_word, 4 * sizeof(uint32_t)));
-        uint32_t check = cap == hipStreamCaptureStatusNone ? maxb * std::max(1u, K.samples) + 1u : iters;
+        uint32_t check = cap == hipStreamCaptureStatusNone ? maxb * std::max(1u, K.samples) + (sun ? 2u : 1u) : iters;
         bool live[4] = {true, true, true, true};
         for (uint32_t it = 0; it < iters; ++it) {
             if (it == check) {
                 for (int h = 0; h < np; ++h)
                     if (live[h])
-                        GK_HIP(hipMemcpyAsync(c.h_word + h, QH[h].cnt + 2 * cur, sizeof(uint32_t), hipMemcpyDeviceToHost,
-                                              ss[h]));
+                        GK_HIP(hipMemcpyAsync(c.h_word + h, QH[h].cnt + 2 * cur, sizeof(uint32_t),
+                                              hipMemcpyDeviceToHost, ss[h]));
                 bool any = false;
                 for (int h = 0; h < np; ++h) {
                     if (!live[h]) continue;
@@ -1393,15 +1456,19 @@ int render_frame(Ctx& c) {
             for (int h = 0; h < np; ++h) {
                 if (!live[h]) continue;
                 c.trace_counter_zeroed[sl[h]] = true;
-                // the trace zeroes the counter of the queue k_ref_shade appends to
+                // the trace zeroes the counters of the queues k_ref_shade appends to
                 const Queues& q = QH[h];
-                st = launch_trace(c, q.o[cur], q.d[cur], q.cnt + 2 * cur, pcount[h], q.hit, q.hit_inst, false,
-                                  q.cnt + 2 * (cur ^ 1), sl[h]);
+                uint32_t* const next = q.cnt + 2 * (cur ^ 1);
+                st = sun ? launch_trace_pair(c, q.o[cur], q.d[cur], q.cnt + 2 * cur, pcount[h], q.hit, q.hit_inst, q.so,
+                                             q.sd, q.cnt + 2 * cur + 1, pcount[h], q.shit, next, sl[h])
+                         : launch_trace(c, q.o[cur], q.d[cur], q.cnt + 2 * cur, pcount[h], q.hit, q.hit_inst, false, next,
+                                        sl[h]);
                 if (st != GK_OK) return st;
             }
             for (int h = 0; h < np; ++h) {
                 if (!live[h]) continue;
-                k_ref_shade<<<nblk(pcount[h]), 256, 0, ss[h]>>>(S0, K, T, QH[h], P, cur, tn[h]);
+                if (sun) k_ref_shade<true><<<nblk(pcount[h]), 256, 0, ss[h]>>>(S0, K, T, QH[h], P, cur, tn[h]);
+                else k_ref_shade<false><<<nblk(pcount[h]), 256, 0, ss[h]>>>(S0, K, T, QH[h], P, cur, tn[h]);
                 GK_HIP(hipGetLastError());
             }
             cur ^= 1;
@@ -1441,7 +1508,7 @@ int render_frame(Ctx& c) {
                 const uint32_t m = pcount[h];
                 if (it + 1 < iters)
                     st = launch_trace_pair(c, q.o[nxt], q.d[nxt], q.cnt + 2 * nxt, m, q.hit, q.hit_inst, q.so, q.sd,
-                                           q.cnt + sh, m, q.shit, sl[h]);
+                                           q.cnt + sh, m, q.shit, nullptr, sl[h]);
                 else
                     st = launch_trace(c, q.so, q.sd, q.cnt + sh, m, q.shit, nullptr, true, nullptr, sl[h]);
                 if (st != GK_OK) return st;

@@ -315,7 +315,9 @@ typedef struct gk_bvh_stats {
 
 /* Per-frame statistics (the reference's SCOPED_GPU_TIMER passes). */
 typedef struct gk_stats {
-    uint64_t rays_traced;      /* primary + extension + shadow rays           */
+    uint64_t rays_traced;      /* primary + extension + shadow rays (REF_V2 with a sun: its sun
+                                  rays are shadow rays, and a path that only waits for one
+                                  counts as an extension ray)                  */
     uint64_t extension_rays;
     uint64_t shadow_rays;
     uint64_t path_vertices;    /* shaded hits                                  */

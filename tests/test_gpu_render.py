@@ -341,3 +341,55 @@ def test_ref_v2_two_pipelines_give_the_single_pipeline_frame():
         assert np.array_equal(a[t].view(np.uint8), c[t].view(np.uint8)), t
     print(f"moving pixels {(a['MOTIONMOMENT'] != 0).mean():.3f}, rays {ra}")
     assert ra > 2 * W * H and a["RADIANCE"][..., :3].max() > 0.1
+
+
+# one to three samples, a single bounce (no sun ray but the pixel's last), dielectric primaries
+# (their own bounce limit, no early exit), fast gather, moved pixels (four times the samples),
+# and a frame split into two pipelines
+@pytest.mark.parametrize("W,H,samples,bounces,max_bounces,flags,moved", [
+    (64, 64, 1, 4, 10, 0, False), (61, 35, 3, 8, 8, 0, False), (32, 32, 2, 1, 1, 0, False),
+    (64, 48, 2, 4, 6, gk.FRAME_FAST_GATHER, False), (40, 40, 1, 3, 5, 0, True), (640, 416, 1, 6, 8, 0, False)])
+def test_ref_v2_sun_rays_match_oracle(W, H, samples, bounces, max_bounces, flags, moved):
+    """REF_V2 frames lit by a sun through the Cornell box's open front: the
+    sun rays of a vertex and of the pixel's end answer as the oracle's, the paths draw the same
+    random numbers, and samples end where the oracle's do."""
+    s = scenes.all_models_cornell()
+    osc = po.OracleScene(s)
+    moment = np.zeros((H, W), np.uint16)
+
+    def params(f, prev=None):
+        p = cornell_params(W, H, frame=f, bounces=bounces, samples=samples, prev=prev)
+        p.max_bounces = max_bounces
+        p.has_sky = p.has_sun = 1
+        p.sky_color[:] = [0.4, 0.5, 0.7, 1.0]
+        p.sun_direction[:] = [0.25, 0.45, -0.857321, 0.0]
+        p.sun_color[:] = [5.0, 4.0, 3.0, 1.0]
+        p.flags |= flags
+        return p
+
+    with gk.Context(W, H) as ctx:
+        ctx.upload(s)
+        prev = None
+        for f in range(3):
+            p = params(f, prev)
+            if moved and f:
+                w = np.eye(4, dtype=np.float32)
+                w[0, 3] = 0.03 * f
+                ctx.update_instances(w[None])
+                osc.update_instances(w[None])
+            ctx.frame(p)
+            ctx.render()
+            ctx.sync()
+            o = osc.render_refv2(p, W, H, moment=moment)
+            gd, gs = ctx.read("SINGLE_DIFFUSE"), ctx.read("SINGLE_SPECULAR")
+            od, os_ = o["diffuse"].astype(np.float16), o["spec"].astype(np.float16)
+            same = np.all(gd.view(np.uint16) == od.view(np.uint16), axis=2) & \
+                np.all(gs.view(np.uint16) == os_.view(np.uint16), axis=2)
+            assert same.mean() > 0.97, (f, same.mean())
+            err = relmse(gd[..., :3].astype(np.float64) + gs[..., :3],
+                         o["diffuse"][..., :3].astype(np.float64) + o["spec"][..., :3])
+            assert err < 1e-3, (f, err)
+            prev = p
+        lit = o["diffuse"][..., :3].max(axis=2) > 1.0
+        assert lit.mean() > 0.02  # the sun reaches the box
+        assert ctx.stats().shadow_rays > W * H
