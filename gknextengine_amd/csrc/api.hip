@@ -344,7 +344,7 @@ int gk_create(const gk_device_desc* desc, gk_ctx** out) {
         delete ctx;
         return GK_ERR_HIP;
     }
-    for (auto& e : c.ev) (void)hipEventCreate(&e);
+    for (auto& e : c.ev) (void)hipEventCreateWithFlags(&e, hipEventDisableSystemFence);
     // gk_trace_static's array on this GPU; a failure is reported by gk_trace_static itself
     (void)static_scratch_init(c.device);
     const int s = alloc_targets(c);
@@ -642,8 +642,8 @@ int gk_target_info(gk_ctx* ctx, int target, size_t* bytes, void** device_ptr) {
     return GK_OK;
 }
 
-// Statistics since the context was created: ray counts from device counters, trace
-// time summed over the HIP events bracketing every trace launch, and the stage times of
+// Statistics since the context was created: ray counts and the trace launches' times from
+// the slots' device words, and the stage times of
 // the last frame (events ev[0..6] of render_frame / post_process).
 int gk_get_stats(gk_ctx* ctx, gk_stats* out) {
     GK_CHECK_CTX_KEEP(ctx);

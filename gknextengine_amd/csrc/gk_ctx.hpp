@@ -130,6 +130,43 @@ struct BuildScratch {
     DevBuf<float> bounds;                 // scene centroid bounds (6 floats as ordered ints)
 };
 
+// Device words of a trace slot, behind its spill stacks. A launch's time is taken by its own
+// waves from the constant-rate clock (its first work-group's start; the latest end over the
+// waves that traced, in one of 64 words on lines of their own) and added to `ticks` by the
+// kernel that readies the slot for the next launch. HIP events around each launch cost about
+// 10 us of stream time: a 16-frame 256x256 preview of 6 launches a frame 4.04 -> 3.41 ms, four
+// 1080p city frames of 24 launches each 11.2 -> 10.8 ms.
+constexpr int kTraceEnds = 64;
+struct TraceSlot {
+    uint32_t next;                // the next ray to fetch
+    uint32_t overflow;            // a traversal stack overflowed
+    unsigned long long rays[2];   // rays traced: closest hit, occlusion
+    unsigned long long start;     // of the launch whose time is not in `ticks` yet (0: none)
+    unsigned long long ticks;     // of the launches before it
+    uint32_t pad0[22];
+    struct { unsigned long long t; uint32_t pad[30]; } end[kTraceEnds];
+};
+static_assert(sizeof(TraceSlot) == 128 * (kTraceEnds + 1), "one line each");
+
+// Readies a slot for its next launch; run by the 64 lanes of one wave, in a kernel between
+// the slot's launches.
+__device__ inline void trace_slot_next(TraceSlot* s) {
+    unsigned long long t = s->end[threadIdx.x & 63u].t;
+#pragma unroll
+    for (int k = 32; k >= 1; k >>= 1) {
+        const unsigned long long o = __shfl_xor(t, k);
+        t = o > t ? o : t;
+    }
+    if ((threadIdx.x & 63u) == 0u) {
+        const unsigned long long t0 = s->start;
+        s->next = 0u;
+        if (t0 != 0ull) {
+            if (t > t0) s->ticks += t - t0;
+            s->start = 0ull;
+        }
+    }
+}
+
 // ------------------------------------------------------------------ context
 struct Ctx {
     int device = 0;
@@ -259,16 +296,14 @@ struct Ctx {
         DevBuf<float4> s_dir;                 // current ray direction
         DevBuf<float4> s_ppos, s_pnrm, s_palb;  // primary vertex, its (textured) albedo
         DevBuf<ushort4> hist_d, hist_s, hist_a;  // previous accumulation targets (RGBA16F)
-        DevBuf<uint32_t> spill;               // traversal stack overflow, then the launch counters
+        DevBuf<uint32_t> spill;               // traversal stack overflow, then the slot's TraceSlot
         DevBuf<uint32_t> pspill[3];           // the same for trace slots 1..3
-        uint32_t spill_threads = 0;
     } wf;
 
-    // timing: per-launch trace events (collected after a stream synchronisation)
+    // stage times of the last frame; like the fork and join events without a system-scope fence
+    // (only this device's streams and its clock use them, and a fence writes every L2 back):
+    // the preview above 3.47 -> 3.32 ms, the city frames 10.9 -> 10.7 ms
     hipEvent_t ev[16] = {};
-    std::vector<std::pair<hipEvent_t, hipEvent_t>> tev;
-    uint32_t tev_used = 0;
-    uint64_t trace_launches = 0;
     bool stack_overflow = false;        // a traversal stack overflowed since gk_get_stats last reported
     bool trace_counter_zeroed[4] = {};  // per slot: the next launch's counter is already 0
     bool trace_split = false;           // a frame's two path pipelines are being enqueued
@@ -310,11 +345,10 @@ int launch_trace_pair(Ctx& c, const float4* o, const float4* d, const uint32_t* 
                       float4* hit, uint32_t* hit_inst, const float4* so, const float4* sd,
                       const uint32_t* scount_dev, uint32_t smax_count, float4* shit, uint32_t* clear, int slot = 0);
 int launch_trace_user(Ctx& c, const gk_ray* rays, uint32_t n, gk_hit* hits, uint32_t* inst, uint32_t flags);
-// the ray counter a trace launch in `slot` starts from (allocates the slot's spill area); a
-// caller whose kernel zeroed it sets Ctx::trace_counter_zeroed[slot], and the next launch in
-// that slot skips its reset
-uint32_t* trace_counter(Ctx& c, int slot = 0);
-int ensure_spill(Ctx& c, uint32_t threads, int slot = 0);
+// the words a trace launch in `slot` starts from (allocates the slot's spill area); a caller
+// whose kernel ran trace_slot_next on them sets Ctx::trace_counter_zeroed[slot], and the next
+// launch in that slot skips its own
+TraceSlot* trace_slot(Ctx& c, int slot = 0);
 int collect_timing(Ctx& c);
 // gk_trace_static's device array: resolved per GPU by gk_create; the overflow flag of the
 // last call on c's GPU, read and cleared

@@ -27,7 +27,6 @@
 
 namespace gk {
 
-int collect_timing(Ctx& c);
 
 namespace {
 
@@ -417,17 +416,6 @@ GridK grid_k(const Ctx& c) {
     return k;
 }
 
-// keep room for the trace launches' timing events (folded into the frame statistics)
-int reserve_trace_events(Ctx& c) {
-    if (c.tev_used + 64u > c.tev.size() && c.tev_used > 0) {
-        // the recorded launches may be on any slot's stream
-        GK_HIP(hipStreamSynchronize(c.stream));
-        for (auto& ps : c.pstream) if (ps) GK_HIP(hipStreamSynchronize(ps));
-        return collect_timing(c);
-    }
-    return GK_OK;
-}
-
 }  // namespace
 
 ProbeDev probe_dev(const Ctx& c) {
@@ -465,8 +453,7 @@ int probes_init(Ctx& c, const gk_probe_grid& g) {
 int probes_voxelize(Ctx& c) {
     auto& P = c.probes;
     if (P.count == 0 || !c.scene_ready) return GK_ERR_STATE;
-    int st = reserve_trace_events(c);
-    if (st != GK_OK) return st;
+    int st = GK_OK;
     const uint32_t chunk = std::min(kChunk, P.count);
     auto& W = P.w[0];
     const size_t nr = size_t(chunk) * kVoxRays;
@@ -485,8 +472,6 @@ int probes_voxelize(Ctx& c) {
         k_vox_finish<<<nblk(n), 256, 0, c.stream>>>(s, g, first, n, W.rd.ptr, W.hit.ptr, W.hit_inst.ptr,
                                                     c.tri_rec.ptr, P.voxels.ptr);
         GK_HIP(hipGetLastError());
-        st = reserve_trace_events(c);
-        if (st != GK_OK) return st;
     }
     return GK_OK;
 }
@@ -496,8 +481,7 @@ int probes_bake(Ctx& c, uint32_t first, uint32_t count) {
     if (P.count == 0 || !c.scene_ready || !c.frame_ready) return GK_ERR_STATE;
     if (first > P.count || count > P.count - first) return GK_ERR_ARG;
     if (count == 0) return GK_OK;
-    int st = reserve_trace_events(c);
-    if (st != GK_OK) return st;
+    int st = GK_OK;
     const gk_frame_params& fp = c.params;
     BakeK K{};
     K.g = grid_k(c);
@@ -539,14 +523,14 @@ int probes_bake(Ctx& c, uint32_t first, uint32_t count) {
         GK_HIP(W.so.resize(std::max(W.so.count, ns)));
         GK_HIP(W.sd.resize(std::max(W.sd.count, ns)));
         GK_HIP(W.shit.resize(std::max(W.shit.count, ns)));
-        if (!trace_counter(c, h)) return GK_ERR_OOM;  // a slot's first use clears its counters on `stream`
+        if (!trace_slot(c, h)) return GK_ERR_OOM;  // a slot's first use clears its words on `stream`
     }
     hipStream_t ss[2] = {c.stream, c.stream};
     if (two) {
-        if (!c.fork_ev) GK_HIP(hipEventCreateWithFlags(&c.fork_ev, hipEventDisableTiming));
+        if (!c.fork_ev) GK_HIP(hipEventCreateWithFlags(&c.fork_ev, hipEventDisableTiming | hipEventDisableSystemFence));
         if (!c.pstream[0]) {
             GK_HIP(hipStreamCreateWithFlags(&c.pstream[0], hipStreamNonBlocking));
-            GK_HIP(hipEventCreateWithFlags(&c.join_ev[0], hipEventDisableTiming));
+            GK_HIP(hipEventCreateWithFlags(&c.join_ev[0], hipEventDisableTiming | hipEventDisableSystemFence));
         }
         ss[1] = c.pstream[0];
         GK_HIP(hipEventRecord(c.fork_ev, c.stream));
@@ -580,8 +564,6 @@ int probes_bake(Ctx& c, uint32_t first, uint32_t count) {
         k_bake_commit<<<nblk(n), 256, 0, st_h>>>(W.list.ptr, W.counters.ptr, P.cubes.ptr, W.face_sky.ptr,
                                                  P.next.ptr, P.voxels.ptr);
         GK_HIP(hipGetLastError());
-        st = reserve_trace_events(c);
-        if (st != GK_OK) return st;
         h = two ? h ^ 1 : 0;
     }
     c.trace_split = false;

@@ -89,6 +89,7 @@ struct TraceJob {
     uint32_t* inst;                  // closest: instance of the hit (may be null)
     uint32_t* clear;                 // a counter other than count_dev the launch sets to 0 (may be
                                      // null): the queue the shading after the trace appends to
+    uint32_t shift;                  // 1: o and d are the halves of gk_ray records (d = o + 1)
 };
 
 // MODE 0: one closest-hit job; 1: one any-hit job; 2: a closest-hit job then an any-hit
@@ -307,8 +308,8 @@ __device__ void trace_quads(const Bvh4Node* __restrict__ blas, const TriRec* __r
         const bool second = MODE == 2 && r >= c0;
         const uint32_t ri = second ? r - c0 : r;
         const bool any = MODE == 1 || second;
-        const float4 o = second ? j1.o[ri] : j0.o[ri];
-        const float4 d = second ? j1.d[ri] : j0.d[ri];
+        const float4 o = second ? j1.o[ri] : j0.o[ri << j0.shift];
+        const float4 d = second ? j1.d[ri] : j0.d[ri << j0.shift];
         const f3 wO = ld3(o), wD = ld3(d);
         const f3 wrD = f3{safercp(wD.x), safercp(wD.y), safercp(wD.z)};
         f3 O = wO, D = wD, rD = wrD;
@@ -439,8 +440,9 @@ __global__ __launch_bounds__(kBlock) void k_trace(
     const Bvh4Node* __restrict__ blas, const TriRec* __restrict__ tris,
     const Bvh4Node* __restrict__ tlas, const uint32_t* __restrict__ tlas_prims,
     const InstDev* __restrict__ inst, uint32_t blas_root, TraceJob j0, TraceJob j1,
-    uint32_t* __restrict__ next_ray, uint32_t* __restrict__ spill,
-    uint32_t* __restrict__ overflow_flag, unsigned long long* __restrict__ ray_stats) {
+    TraceSlot* __restrict__ slot, uint32_t* __restrict__ spill) {
+    uint32_t* const next_ray = &slot->next;
+    uint32_t* const overflow_flag = &slot->overflow;
     __shared__ uint32_t lds[kLdsWords];
     auto ring = reinterpret_cast<uint32_t (*)[kBlock]>(lds);
     const uint32_t stride = gridDim.x * kBlock;
@@ -453,14 +455,20 @@ __global__ __launch_bounds__(kBlock) void k_trace(
     }
     const uint32_t count = c0 + c1;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
+        slot->start = wall_clock64();
         if (j0.clear) *j0.clear = 0u;
         if (MODE == 2 && j1.clear) *j1.clear = 0u;
-        atomicAdd(&ray_stats[MODE == 1 ? 1 : 0], (unsigned long long)c0);
-        if (MODE == 2) atomicAdd(&ray_stats[1], (unsigned long long)c1);
+        atomicAdd(&slot->rays[MODE == 1 ? 1 : 0], (unsigned long long)c0);
+        if (MODE == 2) atomicAdd(&slot->rays[1], (unsigned long long)c1);
     }
+    auto stamp_end = [&]() {  // this wave is done
+        if (__lane_id() == 0u)
+            atomicMax(&slot->end[(gtid >> 6) % uint32_t(kTraceEnds)].t, (unsigned long long)wall_clock64());
+    };
     if (count <= (TWO ? kQuadRaysTwo : kQuadRays) * gridDim.x * kQuads) {
         trace_quads<MODE, TWO>(blas, tris, tlas, tlas_prims, inst, blas_root, j0, j1, c0, count,
                                reinterpret_cast<uint32_t (*)[kQuads]>(lds), overflow_flag);
+        if ((gtid & ~63u) / 4u < count) stamp_end();  // a wave without a ray says nothing
         return;
     }
     // rays a wave holds at once: its share of the launch. The launch holds more rays than the
@@ -498,8 +506,8 @@ __global__ __launch_bounds__(kBlock) void k_trace(
                     if (rank < n_take && r < count) {
                         const bool second = MODE == 2 && r >= c0;
                         const uint32_t ri = second ? r - c0 : r;
-                        const float4 o = second ? j1.o[ri] : j0.o[ri];
-                        const float4 d = second ? j1.d[ri] : j0.d[ri];
+                        const float4 o = second ? j1.o[ri] : j0.o[ri << j0.shift];
+                        const float4 d = second ? j1.d[ri] : j0.d[ri << j0.shift];
                         L.ray = ri;
                         L.job1 = second;
                         L.any = MODE == 1 || second;
@@ -685,11 +693,17 @@ __global__ __launch_bounds__(kBlock) void k_trace(
             L.node = kNone;
         }
     }
+    stamp_end();
 }
 
-__global__ void k_reset_counter(uint32_t* p) { *p = 0u; }
+__global__ void k_clear_words(uint32_t* __restrict__ p, uint32_t n) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] = 0u;
+}
 
-// user gk_ray/gk_hit records <-> queue layout
+__global__ __launch_bounds__(64) void k_slot_next(TraceSlot* s) { trace_slot_next(s); }
+
+// user gk_ray records -> queue layout
 __global__ void k_unpack_rays(const gk_ray* __restrict__ r, uint32_t n, float4* o, float4* d) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -720,61 +734,42 @@ uint32_t persistent_blocks(int device, K kern, int cap = kMaxBlocksPerCU) {
 
 }  // namespace
 
-int ensure_spill(Ctx& c, uint32_t threads, int slot) {
-    const size_t need = size_t(threads) * kSpill;
-    DevBuf<uint32_t>& sp = slot ? c.wf.pspill[slot - 1] : c.wf.spill;
-    if (sp.count < need + 8) {
-        GK_HIP(sp.resize(need + 8));
-        GK_HIP(hipMemsetAsync(sp.ptr + need, 0, 32, c.stream));
-    }
-    c.wf.spill_threads = threads;
-    if (c.tev.empty()) {
-        c.tev.resize(1024);
-        for (auto& e : c.tev) {
-            GK_HIP(hipEventCreate(&e.first));
-            GK_HIP(hipEventCreate(&e.second));
-        }
-    }
-    return GK_OK;
-}
+// threads of the largest grid: a slot's spill area is laid out for it, so the TraceSlot behind
+// it never moves
+static uint32_t spill_threads(const Ctx& c) { return cu_count(c.device) * kMaxBlocksPerCU * kBlock; }
 
-uint32_t* trace_counter(Ctx& c, int slot) {
-    // the spill area is laid out for the largest grid, so its tail (counters) never moves.
-    // A slot's area is allocated (and its counters cleared on `stream`) on first use.
-    const uint32_t cap_threads = cu_count(c.device) * kMaxBlocksPerCU * kBlock;
-    if (ensure_spill(c, cap_threads, slot) != GK_OK) return nullptr;
-    const DevBuf<uint32_t>& sp = slot ? c.wf.pspill[slot - 1] : c.wf.spill;
-    return sp.ptr + size_t(cap_threads) * kSpill;  // [next ray, overflow, stats u64 x2]
+TraceSlot* trace_slot(Ctx& c, int slot) {
+    // a slot's area is allocated (and its words cleared on `stream`) on first use
+    const size_t words = size_t(spill_threads(c)) * kSpill;  // a whole number of 128-byte lines
+    DevBuf<uint32_t>& sp = slot ? c.wf.pspill[slot - 1] : c.wf.spill;
+    if (sp.count == 0) {
+        constexpr uint32_t tail = sizeof(TraceSlot) / 4;
+        if (sp.resize(words + tail) != hipSuccess) return nullptr;
+        k_clear_words<<<(tail + 255) / 256, 256, 0, c.stream>>>(sp.ptr + words, tail);
+        if (hipGetLastError() != hipSuccess) return nullptr;
+    }
+    return reinterpret_cast<TraceSlot*>(sp.ptr + words);
 }
 
 // Launches one persistent trace over up to two jobs (mode as k_trace) in a slot (its stream
-// and spill area). Each launch is bracketed by HIP events on that stream (collected by
-// collect_timing).
+// and spill area).
 static int launch_jobs(Ctx& c, int mode, const TraceJob& j0, const TraceJob& j1, int slot) {
-    const bool zeroed = c.trace_counter_zeroed[slot];  // applies to this launch only
+    const bool ready = c.trace_counter_zeroed[slot];  // applies to this launch only
     c.trace_counter_zeroed[slot] = false;
-    uint32_t* tail = trace_counter(c, slot);
-    if (!tail) return GK_ERR_OOM;
+    TraceSlot* ts = trace_slot(c, slot);
+    if (!ts) return GK_ERR_OOM;
     hipStream_t st = slot ? c.pstream[slot - 1] : c.stream;
     uint32_t* spill = slot ? c.wf.pspill[slot - 1].ptr : c.wf.spill.ptr;
-    uint32_t* next = tail;
-    uint32_t* ovf = tail + 1;
-    unsigned long long* rs = reinterpret_cast<unsigned long long*>(tail + 2);
-    if (!zeroed) k_reset_counter<<<1, 1, 0, st>>>(next);
+    if (!ready) k_slot_next<<<1, 64, 0, st>>>(ts);
     const bool two = !c.blas_only;
     const uint32_t root = c.h_meshes.empty() ? 0u : c.h_meshes[0].root;
-    const Bvh4Node* tl = c.tlas_nodes.ptr;
     auto* kern = mode == 0 ? (two ? k_trace<0, true> : k_trace<0, false>)
                : mode == 1 ? (two ? k_trace<1, true> : k_trace<1, false>)
                            : (two ? k_trace<2, true> : k_trace<2, false>);
     const uint32_t blocks = persistent_blocks(c.device, kern, c.trace_split ? kSplitBlocksPerCU : kMaxBlocksPerCU);
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    if (c.tev_used < c.tev.size()) { e0 = c.tev[c.tev_used].first; e1 = c.tev[c.tev_used].second; c.tev_used++; }
-    if (e0) GK_HIP(hipEventRecord(e0, st));
-    kern<<<blocks, kBlock, 0, st>>>(c.blas_nodes.ptr, c.tris.ptr, tl, c.tlas_prims.ptr, c.inst.ptr, root, j0, j1,
-                                   next, spill, ovf, rs);
+    kern<<<blocks, kBlock, 0, st>>>(c.blas_nodes.ptr, c.tris.ptr, c.tlas_nodes.ptr, c.tlas_prims.ptr, c.inst.ptr, root,
+                                   j0, j1, ts, spill);
     GK_HIP(hipGetLastError());
-    if (e1) GK_HIP(hipEventRecord(e1, st));
     return GK_OK;
 }
 
@@ -784,7 +779,7 @@ static int launch_jobs(Ctx& c, int mode, const TraceJob& j0, const TraceJob& j1,
 int launch_trace(Ctx& c, const float4* ray_o, const float4* ray_d, const uint32_t* count_dev,
                  uint32_t max_count, float4* hit, uint32_t* hit_inst, bool any_hit, uint32_t* clear, int slot) {
     if (max_count == 0) return GK_OK;
-    const TraceJob j0{ray_o, ray_d, count_dev, max_count, hit, any_hit ? nullptr : hit_inst, clear};
+    const TraceJob j0{ray_o, ray_d, count_dev, max_count, hit, any_hit ? nullptr : hit_inst, clear, 0u};
     return launch_jobs(c, any_hit ? 1 : 0, j0, TraceJob{}, slot);
 }
 
@@ -793,70 +788,86 @@ int launch_trace(Ctx& c, const float4* ray_o, const float4* ray_d, const uint32_
 int launch_trace_pair(Ctx& c, const float4* o, const float4* d, const uint32_t* count_dev, uint32_t max_count,
                       float4* hit, uint32_t* hit_inst, const float4* so, const float4* sd,
                       const uint32_t* scount_dev, uint32_t smax_count, float4* shit, uint32_t* clear, int slot) {
-    const TraceJob j0{o, d, count_dev, max_count, hit, hit_inst, clear};
-    const TraceJob j1{so, sd, scount_dev, smax_count, shit, nullptr, clear ? clear + 1 : nullptr};
+    const TraceJob j0{o, d, count_dev, max_count, hit, hit_inst, clear, 0u};
+    const TraceJob j1{so, sd, scount_dev, smax_count, shit, nullptr, clear ? clear + 1 : nullptr, 0u};
     return launch_jobs(c, 2, j0, j1, slot);
 }
 
-// Sums the elapsed time of the trace launches recorded since the last call (the stream
-// must have been synchronised) and reads the device ray counters.
+// Reads every slot's words into the statistics (the streams must have been synchronised):
+// rays and trace time since the context was created, overflow flags.
 int collect_timing(Ctx& c) {
-    for (uint32_t i = 0; i < c.tev_used; ++i) {
-        float ms = 0.f;
-        GK_HIP(hipEventElapsedTime(&ms, c.tev[i].first, c.tev[i].second));
-        c.stats.ms_trace += ms;
-        c.trace_launches++;
-    }
-    c.tev_used = 0;
-    if (c.wf.spill_threads) {
-        // every slot's counters: rays since the spill areas were allocated, overflow flags
-        c.stats.rays_traced = 0;
-        c.stats.shadow_rays = 0;
-        for (int slot = 0; slot < 4; ++slot) {
-            const DevBuf<uint32_t>& sp = slot ? c.wf.pspill[slot - 1] : c.wf.spill;
-            if (!sp.ptr) continue;
-            unsigned long long v[2] = {0, 0};
-            uint32_t ovf = 0;
-            const uint32_t* tail = sp.ptr + size_t(c.wf.spill_threads) * kSpill;
-            GK_HIP(hipMemcpy(v, tail + 2, 16, hipMemcpyDeviceToHost));
-            GK_HIP(hipMemcpy(&ovf, tail + 1, 4, hipMemcpyDeviceToHost));
-            c.stats.rays_traced += v[0] + v[1];
-            c.stats.shadow_rays += v[1];
-            if (ovf) {  // kept until gk_get_stats reports it; the device flag starts over
-                c.stack_overflow = true;
-                const uint32_t zero = 0;
-                GK_HIP(hipMemcpy(const_cast<uint32_t*>(tail + 1), &zero, 4, hipMemcpyHostToDevice));
-            }
+    int khz = 0;
+    GK_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, c.device));
+    c.stats.rays_traced = 0;
+    c.stats.shadow_rays = 0;
+    unsigned long long ticks = 0;
+    for (int slot = 0; slot < 4; ++slot) {
+        const DevBuf<uint32_t>& sp = slot ? c.wf.pspill[slot - 1] : c.wf.spill;
+        if (!sp.ptr) continue;
+        TraceSlot* ts = trace_slot(c, slot);
+        TraceSlot h;
+        GK_HIP(hipMemcpy(&h, ts, sizeof(h), hipMemcpyDeviceToHost));
+        c.stats.rays_traced += h.rays[0] + h.rays[1];
+        c.stats.shadow_rays += h.rays[1];
+        unsigned long long end = 0;  // of the last launch, whose time is not in h.ticks yet
+        for (const auto& e : h.end) end = std::max(end, e.t);
+        ticks += h.ticks + (h.start != 0 && end > h.start ? end - h.start : 0);
+        if (h.overflow) {  // kept until gk_get_stats reports it; the device flag starts over
+            c.stack_overflow = true;
+            const uint32_t zero = 0;
+            GK_HIP(hipMemcpy(&ts->overflow, &zero, 4, hipMemcpyHostToDevice));
         }
     }
+    if (khz > 0) c.stats.ms_trace = double(ticks) / double(khz);
     return GK_OK;
+}
+
+// [a, a + an) and [b, b + bn) share a byte
+static bool overlap(const void* a, size_t an, const void* b, size_t bn) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return x < y + bn && y < x + an;
+}
+
+// Whether a launch may read the caller's gk_ray records where they lie: they are aligned for
+// 16-byte loads and no result overwrites a ray that is still to be read. Other rays are copied
+// to a queue first (a pass of 64 bytes a ray: 20 us of 1.15 ms for a million bulk rays).
+static bool rays_in_place(const gk_ray* rays, uint32_t n, const gk_hit* hits, const uint32_t* inst) {
+    const size_t rb = size_t(n) * sizeof(gk_ray);
+    return reinterpret_cast<uintptr_t>(rays) % 16 == 0 && !overlap(rays, rb, hits, size_t(n) * sizeof(gk_hit)) &&
+           !(inst && overlap(rays, rb, inst, size_t(n) * 4));
 }
 
 int launch_trace_user(Ctx& c, const gk_ray* rays, uint32_t n, gk_hit* hits, uint32_t* inst, uint32_t flags) {
     if (n == 0) return GK_OK;
-    // staging in the wavefront queue 0 (grown on demand)
-    auto& w = c.wf;
-    if (w.ray_o[0].count < n) { GK_HIP(w.ray_o[0].resize(n)); GK_HIP(w.ray_d[0].resize(n)); }
-    k_unpack_rays<<<(n + 255) / 256, 256, 0, c.stream>>>(rays, n, w.ray_o[0].ptr, w.ray_d[0].ptr);
-    GK_HIP(hipGetLastError());
-    static_assert(sizeof(gk_hit) == sizeof(float4), "gk_hit is a float4");
-    return launch_trace(c, w.ray_o[0].ptr, w.ray_d[0].ptr, nullptr, n, reinterpret_cast<float4*>(hits), inst,
-                        (flags & GK_TRACE_ANY) != 0, nullptr);
+    static_assert(sizeof(gk_hit) == sizeof(float4) && sizeof(gk_ray) == 2 * sizeof(float4), "float4 records");
+    const bool any = (flags & GK_TRACE_ANY) != 0;
+    TraceJob j0{reinterpret_cast<const float4*>(rays), reinterpret_cast<const float4*>(rays) + 1, nullptr, n,
+                reinterpret_cast<float4*>(hits), any ? nullptr : inst, nullptr, 1u};
+    if (n > 0x7fffffffu || !rays_in_place(rays, n, hits, any ? nullptr : inst)) {
+        // staging in the wavefront queue 0 (grown on demand)
+        auto& w = c.wf;
+        if (w.ray_o[0].count < n) { GK_HIP(w.ray_o[0].resize(n)); GK_HIP(w.ray_d[0].resize(n)); }
+        k_unpack_rays<<<(n + 255) / 256, 256, 0, c.stream>>>(rays, n, w.ray_o[0].ptr, w.ray_d[0].ptr);
+        GK_HIP(hipGetLastError());
+        j0.o = w.ray_o[0].ptr;
+        j0.d = w.ray_d[0].ptr;
+        j0.shift = 0u;
+    }
+    return launch_jobs(c, any ? 1 : 0, j0, TraceJob{}, 0);
 }
 
 // ---------------------------------------------------------------- allocation-free ray cast
 // gk_trace_static: the same launch as gk_trace with everything beyond the caller's rays
 // and hits in `scratch`, a static device array that each GPU holds from the library's load
-// to the process's end. Layout (32-bit words): a 64-word head (next ray, overflow flag,
-// two 64-bit ray counts), ray staging (origin/tmin then direction/tmax, float4 each, for
-// kStaticMaxRays rays), then the spill stacks of a kStaticBlocks-work-group launch
-// ([entry][thread], kSpill entries per thread). 24 MiB + 256 bytes.
+// to the process's end. Layout (32-bit words): a TraceSlot, ray staging (origin/tmin then
+// direction/tmax, float4 each, for kStaticMaxRays rays), then the spill stacks of a
+// kStaticBlocks-work-group launch ([entry][thread], kSpill entries per thread). 24 MiB + 8 KiB.
 // Host code never passes `scratch` itself to a kernel (on the host it names a shadow
 // variable, not device memory): gk_create resolves its device address once per GPU with
 // hipGetSymbolAddress, with that GPU current, and every use below goes through it.
 constexpr uint32_t kStaticMaxRays = GK_TRACE_STATIC_MAX_RAYS;
 constexpr uint32_t kStaticBlocks = 256;  // work-groups of a launch (the spill area is sized for it)
-constexpr size_t kStaticHead = 64;
+constexpr size_t kStaticHead = sizeof(TraceSlot) / 4;
 constexpr size_t kStaticWords = kStaticHead + size_t(kStaticMaxRays) * 8 + size_t(kStaticBlocks) * kBlock * kSpill;
 static __device__ __align__(256) uint32_t scratch[kStaticWords];
 
@@ -864,11 +875,6 @@ namespace {
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 uint32_t* g_scratch[kMaxDevices] = {};
-
-__global__ void k_clear_words(uint32_t* __restrict__ p, uint32_t n) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0u;
-}
 }  // namespace
 
 // Resolves this GPU's copy of `scratch` (the caller has made `device` current).
@@ -924,24 +930,28 @@ extern "C" int gk_trace_static(gk_ctx* ctx, const gk_ray* d_rays, uint32_t n, gk
         if (s != GK_OK) return s;
     }
     if (n == 0) return GK_OK;
-    uint32_t* head = base;                                   // next ray, overflow, ray counts
+    TraceSlot* head = reinterpret_cast<TraceSlot*>(base);
     float4* so = reinterpret_cast<float4*>(base + kStaticHead);
     float4* sd = so + kStaticMaxRays;
     uint32_t* spill = reinterpret_cast<uint32_t*>(sd + kStaticMaxRays);
     // the previous call's counters are still there: start from zero
-    k_clear_words<<<1, uint32_t(kStaticHead), 0, c.stream>>>(head, uint32_t(kStaticHead));
-    k_unpack_rays<<<(n + 255) / 256, 256, 0, c.stream>>>(d_rays, n, so, sd);
-    GK_HIP(hipGetLastError());
+    k_clear_words<<<1, 64, 0, c.stream>>>(base, 32u);
     const bool any = (flags & GK_TRACE_ANY) != 0;
     const bool two = !c.blas_only;
     const uint32_t root = c.h_meshes.empty() ? 0u : c.h_meshes[0].root;
     auto* kern = any ? (two ? k_trace<1, true> : k_trace<1, false>) : (two ? k_trace<0, true> : k_trace<0, false>);
     uint32_t blocks = persistent_blocks(c.device, kern);
     if (blocks > kStaticBlocks) blocks = kStaticBlocks;
-    const TraceJob j0{so, sd, nullptr, n, reinterpret_cast<float4*>(d_hits), any ? nullptr : d_inst, nullptr};
+    TraceJob j0{reinterpret_cast<const float4*>(d_rays), reinterpret_cast<const float4*>(d_rays) + 1, nullptr, n,
+                reinterpret_cast<float4*>(d_hits), any ? nullptr : d_inst, nullptr, 1u};
+    if (!rays_in_place(d_rays, n, d_hits, j0.inst)) {
+        k_unpack_rays<<<(n + 255) / 256, 256, 0, c.stream>>>(d_rays, n, so, sd);
+        j0.o = so;
+        j0.d = sd;
+        j0.shift = 0u;
+    }
     kern<<<blocks, kBlock, 0, c.stream>>>(c.blas_nodes.ptr, c.tris.ptr, c.tlas_nodes.ptr, c.tlas_prims.ptr, c.inst.ptr,
-                                         root, j0, TraceJob{}, head, spill, head + 1,
-                                         reinterpret_cast<unsigned long long*>(head + 2));
+                                         root, j0, TraceJob{}, head, spill);
     GK_HIP(hipGetLastError());
     return GK_OK;
 }

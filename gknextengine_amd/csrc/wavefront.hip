@@ -354,12 +354,13 @@ __device__ inline void write_miss_gbuffer(const FrameK& K, const Targets& T, uin
 // queue_state: PT_MIS keeps its per-path state with the queue entries (Queues::q*),
 // REF_V2 in PathState
 // camera rays of paths p_base .. p_base + n - 1 into queue entries 0 .. n - 1; also zeroes the
-// queue counters and the ray counter of the trace launch that follows (trace_next)
+// queue counters and readies the slot of the trace launch that follows
 __global__ void k_raygen(FrameK K, Queues Q, PathState S, uint32_t n, uint32_t queue_state, uint32_t p_base,
-                         uint32_t* __restrict__ trace_next) {
+                         TraceSlot* __restrict__ tslot) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     // queue 0 (word 0) holds the n primary rays; queue 1 (word 2) and both shadow sizes are 0
-    if (i == 0) { Q.cnt[0] = n; Q.cnt[1] = 0u; Q.cnt[2] = 0u; Q.cnt[3] = 0u; *trace_next = 0u; }
+    if (i == 0) { Q.cnt[0] = n; Q.cnt[1] = 0u; Q.cnt[2] = 0u; Q.cnt[3] = 0u; }
+    if (blockIdx.x == 0u && threadIdx.x < 64u) trace_slot_next(tslot);
     if (i >= n) return;
     const uint32_t p = p_base + i;
     const uint32_t px = pixel_of(K, p);
@@ -561,11 +562,14 @@ __device__ inline void ref_end_sample(const DScene& s, const FrameK& K, const Ta
     }
 }
 
-// trace_next: the ray counter of the trace launch that follows, zeroed here
+// tslot: the slot of the trace launch that follows, readied here
 __global__ __launch_bounds__(256) void k_ref_primary(DScene s, FrameK K, Targets T, Queues Q, PathState S,
-                                                     uint32_t* __restrict__ trace_next) {
+                                                     TraceSlot* __restrict__ tslot) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0u) *trace_next = 0u;
+    if (blockIdx.x == gridDim.x - 1u) {  // a work-group of its own
+        if (threadIdx.x < 64u) trace_slot_next(tslot);
+        return;
+    }
     const uint32_t n = Q.cnt[0];
     const bool live = i < n;
     bool emit = false;
@@ -635,7 +639,7 @@ __global__ __launch_bounds__(256) void k_ref_primary(DScene s, FrameK K, Targets
 }
 
 // GetRayColor after the trace (Shading.slang:1039-1081) and the Render loop body
-// (Shading.slang:1117-1171); cur = queue the hits belong to; trace_next as k_ref_primary.
+// (Shading.slang:1117-1171); cur = queue the hits belong to; tslot as k_ref_primary.
 // SUN: sun rays (a vertex's, and the one that ends a pixel) go to the occlusion queue of the
 // bounce, traced in one launch with its extension rays; the path's extension entry finds its
 // answer in the next launch (slot in S.dir's w). The vertex goes on as if the sun were hidden,
@@ -649,9 +653,12 @@ __global__ __launch_bounds__(256) void k_ref_primary(DScene s, FrameK K, Targets
 // dependent loads, 25 to 80 us each. Four waves per SIMD instead of three spill: 14.0 ms.)
 template <bool SUN>
 __global__ __launch_bounds__(256) void k_ref_shade(DScene s, FrameK K, Targets T, Queues Q, PathState S, int cur,
-                                                   uint32_t* __restrict__ trace_next) {
+                                                   TraceSlot* __restrict__ tslot) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0u) *trace_next = 0u;
+    if (blockIdx.x == gridDim.x - 1u) {  // a work-group of its own
+        if (threadIdx.x < 64u) trace_slot_next(tslot);
+        return;
+    }
     const uint32_t n = Q.cnt[2 * cur];
     const int nxt = cur ^ 1;
     const bool live = i < n;
@@ -791,9 +798,12 @@ __global__ __launch_bounds__(256) void k_ref_shade(DScene s, FrameK K, Targets T
 // bit10 last vertex was delta (or camera), bits 16-27 sample index
 // sh: the shadow queue's counter word, 2 nxt + 1 (3 and 1 alternate between bounces)
 __global__ __launch_bounds__(256) void k_pt_shade(DScene s, FrameK K, Targets T, Queues Q, PathState S, int cur,
-                                                  int sh, uint32_t* __restrict__ trace_next) {
+                                                  int sh, TraceSlot* __restrict__ tslot) {
     const uint32_t i0 = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i0 == 0u) *trace_next = 0u;  // the ray counter of the trace launch that follows
+    if (blockIdx.x == gridDim.x - 1u) {  // a work-group of its own readies the slot of the trace that follows
+        if (threadIdx.x < 64u) trace_slot_next(tslot);
+        return;
+    }
     const uint32_t n = Q.cnt[2 * cur];
     const int nxt = cur ^ 1;
     bool emit = false, emit_sh = false;
@@ -1256,12 +1266,6 @@ int render_frame(Ctx& c) {
     auto& w = c.wf;
     hipStream_t s = c.stream;
     const uint32_t n = c.width * c.height;
-    if (c.tev_used + 256u > c.tev.size() && c.tev_used > 0) {
-        // keep room for this frame's trace events: fold the recorded ones into the totals
-        GK_HIP(hipStreamSynchronize(s));
-        st = collect_timing(c);
-        if (st != GK_OK) return st;
-    }
     hipEventRecord(c.ev[0], s);
     if (c.params.flags & GK_FRAME_POST_ONLY) {  // the caller wrote the rt pass's targets
         hipEventRecord(c.ev[1], s);
@@ -1349,13 +1353,13 @@ int render_frame(Ctx& c) {
     // frame runs on `s` and traces in slot 0
     hipStream_t ss[4] = {s, s, s, s};
     int sl[4] = {0, 0, 0, 0};
-    uint32_t* tn[4] = {nullptr, nullptr, nullptr, nullptr};
+    TraceSlot* tn[4] = {nullptr, nullptr, nullptr, nullptr};
     static_assert(kPathParts < 4, "a split frame's pipelines use trace slots 1..kPathParts");
     for (int h = 0; split && h < np; ++h) {
-        if (!c.fork_ev) GK_HIP(hipEventCreateWithFlags(&c.fork_ev, hipEventDisableTiming));
+        if (!c.fork_ev) GK_HIP(hipEventCreateWithFlags(&c.fork_ev, hipEventDisableTiming | hipEventDisableSystemFence));
         if (!c.pstream[h]) {
             GK_HIP(hipStreamCreateWithFlags(&c.pstream[h], hipStreamNonBlocking));
-            GK_HIP(hipEventCreateWithFlags(&c.join_ev[h], hipEventDisableTiming));
+            GK_HIP(hipEventCreateWithFlags(&c.join_ev[h], hipEventDisableTiming | hipEventDisableSystemFence));
         }
         ss[h] = c.pstream[h];
         sl[h] = h + 1;
@@ -1375,10 +1379,10 @@ int render_frame(Ctx& c) {
         if (B.sorted) B.sorted += o;
         B.sort_cnt += 32 * h;
     }
-    // the slots' ray counters (a slot's first use allocates and clears them on `s`, so
-    // before the fork)
+    // the slots' words (a slot's first use allocates and clears them on `s`, so before the
+    // fork)
     for (int h = 0; h < np; ++h) {
-        tn[h] = trace_counter(c, sl[h]);
+        tn[h] = trace_slot(c, sl[h]);
         if (!tn[h]) return GK_ERR_OOM;
     }
     // Early start: ray generation and the primary trace read the queues, path state and
@@ -1418,7 +1422,7 @@ int render_frame(Ctx& c) {
     int cur = 0;
     if (ref) {
         for (int h = 0; h < np; ++h) {
-            k_ref_primary<<<nblk(pcount[h]), 256, 0, ss[h]>>>(S0, K, T, QH[h], P, tn[h]);
+            k_ref_primary<<<nblk(pcount[h]) + 1u, 256, 0, ss[h]>>>(S0, K, T, QH[h], P, tn[h]);
             GK_HIP(hipGetLastError());
         }
         cur = 1;
@@ -1467,8 +1471,8 @@ int render_frame(Ctx& c) {
             }
             for (int h = 0; h < np; ++h) {
                 if (!live[h]) continue;
-                if (sun) k_ref_shade<true><<<nblk(pcount[h]), 256, 0, ss[h]>>>(S0, K, T, QH[h], P, cur, tn[h]);
-                else k_ref_shade<false><<<nblk(pcount[h]), 256, 0, ss[h]>>>(S0, K, T, QH[h], P, cur, tn[h]);
+                if (sun) k_ref_shade<true><<<nblk(pcount[h]) + 1u, 256, 0, ss[h]>>>(S0, K, T, QH[h], P, cur, tn[h]);
+                else k_ref_shade<false><<<nblk(pcount[h]) + 1u, 256, 0, ss[h]>>>(S0, K, T, QH[h], P, cur, tn[h]);
                 GK_HIP(hipGetLastError());
             }
             cur ^= 1;
@@ -1499,7 +1503,7 @@ int render_frame(Ctx& c) {
                     k_sort_scan<<<1, 64, 0, ss[h]>>>(q.sort_cnt);
                     k_sort_scatter<<<nblk(m), 256, 0, ss[h]>>>(q, cur);
                 }
-                k_pt_shade<<<nblk(m), 256, 0, ss[h]>>>(S0, K, T, q, P, cur, sh, tn[h]);
+                k_pt_shade<<<nblk(m) + 1u, 256, 0, ss[h]>>>(S0, K, T, q, P, cur, sh, tn[h]);
                 GK_HIP(hipGetLastError());
                 c.trace_counter_zeroed[sl[h]] = true;
             }

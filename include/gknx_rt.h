@@ -322,7 +322,7 @@ typedef struct gk_stats {
     uint64_t shadow_rays;
     uint64_t path_vertices;    /* shaded hits                                  */
     double ms_tlas;
-    double ms_trace;           /* all trace launches                           */
+    double ms_trace;           /* all trace launches, by the device's clock    */
     double ms_shade;           /* raygen + shade + queue compaction/sort       */
     double ms_reproject;
     double ms_denoise;

@@ -310,3 +310,80 @@ def test_build_sizes_trace_as_the_oracle(device, n):
     o, _ = po.OracleScene(s).trace(rays)
     assert np.array_equal(_u32(h), _u32(o))
     assert np.all(_u32(ho[:, 3]) == 1)
+
+
+@pytest.mark.parametrize("layout", ["aligned", "off by a word", "hits over the rays", "hits over the ray behind",
+                                    "instances over the rays"])
+@pytest.mark.parametrize("static", [False, True])
+def test_ray_buffers_read_in_place_or_copied(device, layout, static):
+    """A launch reads 16-byte aligned rays that no result overwrites where they lie and a copy
+    of all others: every layout gives the oracle's hits, for a small batch (quad traversal), one
+    that is no multiple of a wave, and one that refills its waves."""
+    import torch
+    s = gk.procgen_cornell()
+    p = gk.make_frame_params(scenes.CORNELL_CAM["eye"], scenes.CORNELL_CAM["target"], 512, 320, fov=40.0)
+    cam = po.primary_rays(p, 512, 320)
+    osc = po.OracleScene(s)
+    with gk.Context(32, 32) as ctx:
+        ctx.upload(s)
+        cast = ctx.trace_static if static else ctx.trace
+        for n in (1, 2049, 512 * 320):
+            want = _u32(osc.trace(cam[:n])[0])
+            buf = torch.zeros(n * 8 + 64, dtype=torch.float32, device=device)
+            off = 1 if layout == "off by a word" else 0
+            buf[off:off + n * 8] = torch.from_numpy(np.ascontiguousarray(cam[:n], np.float32)).to(device).reshape(-1)
+            hits = torch.zeros(n * 4, dtype=torch.float32, device=device)
+            inst = torch.zeros(n, dtype=torch.int32, device=device)
+            rp = buf.data_ptr() + 4 * off
+            hp, ip = hits.data_ptr(), inst.data_ptr()
+            if layout == "hits over the rays":
+                hp = rp
+            elif layout == "hits over the ray behind":
+                hp = rp + (n * 8 - 4) * 4
+                buf = torch.cat([buf, buf.new_zeros(n * 4)])
+                rp, hp = buf.data_ptr(), buf.data_ptr() + (n * 8 - 4) * 4
+            elif layout == "instances over the rays":
+                ip = rp
+            torch.cuda.synchronize()
+            cast(rp, n, hp, ip)
+            ctx.sync()
+            if hp == hits.data_ptr():
+                got = hits
+            else:
+                first = (hp - buf.data_ptr()) // 4
+                got = buf[first:first + n * 4]
+            assert np.array_equal(got.cpu().numpy().reshape(-1, 4).view(np.uint32), want), n
+
+
+def test_trace_time_adds_up_over_launches_and_slots(device):
+    """ms_trace: the launches' own clock times, summed; a launch that is not followed by
+    another one is in it, and the sum stays below the wall-clock time of the calls."""
+    import time
+
+    import torch
+    s = gk.procgen_city()
+    W, H = 640, 480  # two path pipelines: three slots with the one of gk_trace
+    p = gk.make_frame_params((60, 40, 60), (0, 5, 0), W, H, fov=50.0)
+    rays = torch.from_numpy(np.ascontiguousarray(po.primary_rays(p, W, H), np.float32)).to(device)
+    hits = torch.zeros((W * H, 4), dtype=torch.float32, device=device)
+    with gk.Context(W, H) as ctx:
+        ctx.upload(s)
+        assert ctx.stats().ms_trace == 0.0
+        torch.cuda.synchronize()
+        last = 0.0
+        for k in range(3):
+            t = time.perf_counter()
+            ctx.trace(rays.data_ptr(), W * H, hits.data_ptr())
+            ctx.sync()
+            t = 1e3 * (time.perf_counter() - t)
+            now = ctx.stats().ms_trace
+            assert 0.01 < now - last < t, (k, now, last, t)
+            assert ctx.stats().ms_trace == now  # reading it changes nothing
+            last = now
+        p.total_frames = 1
+        ctx.frame(p)
+        t = time.perf_counter()
+        ctx.render()
+        ctx.sync()
+        t = 1e3 * (time.perf_counter() - t)
+        assert 0.02 < ctx.stats().ms_trace - last < 2 * t  # two launches run at a time
