@@ -19,6 +19,9 @@ the same-seed render measure it.
 """
 from __future__ import annotations
 
+import ctypes as C
+
+import numpy as np
 import torch
 
 from . import Context, FrameParams, Material, check, lib
@@ -26,16 +29,29 @@ from . import Context, FrameParams, Material, check, lib
 ADJOINT_SEED_XOR = 0x5BD1E995
 
 
+def _materials(base: list[Material], params: torch.Tensor) -> C.Array:
+    """base with albedo / roughness / metallic from params (one copy to the host). The columns
+    are written as a whole: field by field, 257 materials took 0.45 ms, in the render and again
+    in its backward (0.9 of 3.5 ms for 512 x 512 pixels of 4 samples)."""
+    p = params.detach().to("cpu", torch.float32).numpy()[:len(base)]
+    if len(p) < len(base):
+        raise IndexError(f"{len(base)} materials, {len(p)} rows of parameters")
+    mats = (Material * len(base))(*base)
+    words = np.frombuffer(mats, np.float32).reshape(len(base), C.sizeof(Material) // 4)
+    at = Material.diffuse.offset // 4
+    words[:, at:at + 3] = p[:, :3]
+    words[:, Material.fuzziness.offset // 4] = p[:, 3]
+    words[:, Material.metalness.offset // 4] = p[:, 4]
+    return mats
+
+
+def _apply(ctx: Context, mats: C.Array) -> None:
+    check(lib().gk_materials_update(ctx.h, mats, 0, len(mats)), "gk_materials_update")
+
+
 def apply_params(ctx: Context, base: list[Material], params: torch.Tensor) -> None:
     """Writes albedo / roughness / metallic from params into the context's materials."""
-    p = params.detach().to("cpu", torch.float32).numpy()
-    mats = (Material * len(base))()
-    for i, m in enumerate(base):
-        mats[i] = m
-        mats[i].diffuse[0], mats[i].diffuse[1], mats[i].diffuse[2] = (float(v) for v in p[i, :3])
-        mats[i].fuzziness = float(p[i, 3])
-        mats[i].metalness = float(p[i, 4])
-    check(lib().gk_materials_update(ctx.h, mats, 0, len(base)), "gk_materials_update")
+    _apply(ctx, _materials(base, params))
 
 
 def params_of(materials: list[Material]) -> torch.Tensor:
@@ -54,27 +70,28 @@ class _Render(torch.autograd.Function):
     @staticmethod
     def forward(fctx, params, ctx, base, frame, decorrelate):
         _check_params(params, base)
-        apply_params(ctx, base, params)
+        mats = _materials(base, params)
+        _apply(ctx, mats)
         ctx.frame(frame)
         img = torch.empty((ctx.height, ctx.width, 4), dtype=torch.float32, device=params.device)
         torch.cuda.synchronize()
         check(lib().gk_render_radiance(ctx.h, img.data_ptr()), "gk_render_radiance")
         ctx.sync()
-        # what the backward must replay: this call's parameters and frame constants
-        fctx.gk = (ctx, base, params.detach().clone(), FrameParams.from_buffer_copy(frame), bool(decorrelate))
+        # what the backward must replay: this call's materials and frame constants
+        fctx.gk = (ctx, mats, FrameParams.from_buffer_copy(frame), bool(decorrelate))
         return img[..., :3].clone()
 
     @staticmethod
     def backward(fctx, grad_img):
-        ctx, base, params, frame, decorrelate = fctx.gk
-        apply_params(ctx, base, params)
+        ctx, mats, frame, decorrelate = fctx.gk
+        _apply(ctx, mats)
         replay = FrameParams.from_buffer_copy(frame)
         if decorrelate:
             replay.global_seed = (frame.global_seed ^ ADJOINT_SEED_XOR) & 0xFFFFFFFF
         ctx.frame(replay)
         dl = torch.zeros((ctx.height, ctx.width, 4), dtype=torch.float32, device=grad_img.device)
         dl[..., :3] = grad_img
-        grad = torch.empty(tuple(params.shape), dtype=torch.float32, device=grad_img.device)
+        grad = torch.empty((len(mats), 5), dtype=torch.float32, device=grad_img.device)
         torch.cuda.synchronize()
         check(lib().gk_adjoint(ctx.h, dl.data_ptr(), grad.data_ptr()), "gk_adjoint")
         ctx.sync()
