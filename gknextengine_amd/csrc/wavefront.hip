@@ -1428,10 +1428,11 @@ int render_frame(Ctx& c) {
         cur = 1;
         const bool sun = K.has_sun != 0u;
         // worst case: every sample uses all bounces (samples * 4 for moving pixels); a sample
-        // traces at least once, also with no bounces; with a sun the pixel waits once more for
-        // its last sun ray
+        // traces at least once, also with no bounces; with a sun it may wait once for its last
+        // vertex's sun ray, and the pixel once more for its own
         const uint32_t maxb = std::max(1u, std::max(K.bounces, K.max_bounces));
-        const uint32_t iters = maxb * K.samples * 4u + (sun ? 5u : 4u);
+        const uint32_t per = maxb + (sun ? 1u : 0u);
+        const uint32_t iters = per * K.samples * 4u + 4u;
         // A pipeline's loop ends early once the queue it is about to trace is empty: every
         // sample has finished. Reading the counters back costs a synchronisation of the
         // streams, so they are read after the iterations a pixel without motion can take,
@@ -1439,7 +1440,7 @@ int render_frame(Ctx& c) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         GK_HIP(hipStreamIsCapturing(s, &cap));
         if (cap == hipStreamCaptureStatusNone && !c.h_word) GK_HIP(hipHostMalloc(&c.h_word, 4 * sizeof(uint32_t)));
-        uint32_t check = cap == hipStreamCaptureStatusNone ? maxb * std::max(1u, K.samples) + (sun ? 2u : 1u) : iters;
+        uint32_t check = cap == hipStreamCaptureStatusNone ? per * std::max(1u, K.samples) + 1u : iters;
         bool live[4] = {true, true, true, true};
         for (uint32_t it = 0; it < iters; ++it) {
             if (it == check) {
