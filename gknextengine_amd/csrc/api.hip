@@ -363,6 +363,7 @@ int gk_destroy(gk_ctx* ctx) {
     free_targets(c);
     for (auto& e : c.ev) if (e) (void)hipEventDestroy(e);
     if (c.h_word) (void)hipHostFree(c.h_word);
+    for (auto& e : c.moved_ev) if (e) (void)hipEventDestroy(e);
     if (c.fork_ev) (void)hipEventDestroy(c.fork_ev);
     for (auto& e : c.join_ev) if (e) (void)hipEventDestroy(e);
     for (auto& ps : c.pstream) if (ps) (void)hipStreamDestroy(ps);

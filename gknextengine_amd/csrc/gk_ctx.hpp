@@ -307,7 +307,8 @@ struct Ctx {
     bool stack_overflow = false;        // a traversal stack overflowed since gk_get_stats last reported
     bool trace_counter_zeroed[4] = {};  // per slot: the next launch's counter is already 0
     bool trace_split = false;           // a frame's two path pipelines are being enqueued
-    uint32_t* h_word = nullptr;         // pinned host words (one per path pipeline) for counter read-backs
+    uint32_t* h_word = nullptr;         // pinned host words (one per path pipeline): pixels moved, queue sizes
+    hipEvent_t moved_ev[4] = {};        // after the kernel that says whether a pipeline's pixels moved
     gk_stats stats{};
 };
 

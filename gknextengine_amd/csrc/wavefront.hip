@@ -562,9 +562,10 @@ __device__ inline void ref_end_sample(const DScene& s, const FrameK& K, const Ta
     }
 }
 
-// tslot: the slot of the trace launch that follows, readied here
+// tslot: the slot of the trace launch that follows, readied here; moved (host memory, may be
+// null): set to 1 when a pixel has moved and takes four times the samples
 __global__ __launch_bounds__(256) void k_ref_primary(DScene s, FrameK K, Targets T, Queues Q, PathState S,
-                                                     TraceSlot* __restrict__ tslot) {
+                                                     TraceSlot* __restrict__ tslot, uint32_t* __restrict__ moved) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (blockIdx.x == gridDim.x - 1u) {  // a work-group of its own
         if (threadIdx.x < 64u) trace_slot_next(tslot);
@@ -572,7 +573,7 @@ __global__ __launch_bounds__(256) void k_ref_primary(DScene s, FrameK K, Targets
     }
     const uint32_t n = Q.cnt[0];
     const bool live = i < n;
-    bool emit = false;
+    bool emit = false, more = false;
     float4 ro{}, rd{};
     uint32_t p = 0;
     if (live) {
@@ -613,6 +614,7 @@ __global__ __launch_bounds__(256) void k_ref_primary(DScene s, FrameK K, Targets
                 T.radiance[px] = r;
             } else {
                 const uint32_t mult = moment > 0u ? 4u : 1u;
+                more = moment > 0u;
                 uint32_t nsamp = K.samples * mult;
                 if (nsamp < 1u) nsamp = 1u;
                 S.ppos[p] = make_float4(pos.x, pos.y, pos.z, __uint_as_float(mi));
@@ -634,6 +636,9 @@ __global__ __launch_bounds__(256) void k_ref_primary(DScene s, FrameK K, Targets
         }
         S.rng[p] = make_uint4(seed.x, seed.y, seed.z, seed.w);
     }
+    // one store a work-group: they cross the bus
+    if (__syncthreads_or(more) && moved && threadIdx.x == 0u)
+        __hip_atomic_store(moved, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     const uint32_t slot = block_append(&Q.cnt[2], emit);
     if (emit) { Q.o[1][slot] = ro; Q.d[1][slot] = rd; Q.path[1][slot] = p; }
 }
@@ -1421,9 +1426,20 @@ int render_frame(Ctx& c) {
         for (int h = 0; h < np; ++h) GK_HIP(hipStreamWaitEvent(ss[h], c.fork_ev, 0));
     int cur = 0;
     if (ref) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        GK_HIP(hipStreamIsCapturing(s, &cap));
+        const bool eager = cap == hipStreamCaptureStatusNone;
+        if (eager && !c.h_word) {
+            GK_HIP(hipHostMalloc(&c.h_word, 4 * sizeof(uint32_t), hipHostMallocMapped | hipHostMallocCoherent));
+            for (auto& e : c.moved_ev) GK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        }
         for (int h = 0; h < np; ++h) {
-            k_ref_primary<<<nblk(pcount[h]) + 1u, 256, 0, ss[h]>>>(S0, K, T, QH[h], P, tn[h]);
+            // the last frame's kernel that wrote the word has been waited for
+            if (eager) c.h_word[h] = 0u;
+            k_ref_primary<<<nblk(pcount[h]) + 1u, 256, 0, ss[h]>>>(S0, K, T, QH[h], P, tn[h],
+                                                                   eager ? c.h_word + h : nullptr);
             GK_HIP(hipGetLastError());
+            if (eager) GK_HIP(hipEventRecord(c.moved_ev[h], ss[h]));
         }
         cur = 1;
         const bool sun = K.has_sun != 0u;
@@ -1432,18 +1448,27 @@ int render_frame(Ctx& c) {
         // vertex's sun ray, and the pixel once more for its own
         const uint32_t maxb = std::max(1u, std::max(K.bounces, K.max_bounces));
         const uint32_t per = maxb + (sun ? 1u : 0u);
+        const uint32_t still = per * std::max(1u, K.samples) + (sun ? 1u : 0u);  // of a pixel without motion
         const uint32_t iters = per * K.samples * 4u + 4u;
-        // A pipeline's loop ends early once the queue it is about to trace is empty: every
-        // sample has finished. Reading the counters back costs a synchronisation of the
-        // streams, so they are read after the iterations a pixel without motion can take,
-        // then every maxb iterations; a stream under capture runs the worst case.
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        GK_HIP(hipStreamIsCapturing(s, &cap));
-        if (cap == hipStreamCaptureStatusNone && !c.h_word) GK_HIP(hipHostMalloc(&c.h_word, 4 * sizeof(uint32_t)));
-        uint32_t check = cap == hipStreamCaptureStatusNone ? per * std::max(1u, K.samples) + 1u : iters;
+        // A pipeline whose pixels all rest ends after `still` launches: k_ref_primary has told
+        // the host by the time it has queued them, so nothing is read back (reading the queue's
+        // size there left the chip idle for 30 us, of 208 us of a 256x256 preview frame). One
+        // with moving pixels ends early once the queue it is about to trace is empty. Reading
+        // the counters back costs a synchronisation of the streams, so they are read after
+        // `still` launches, then every maxb; a stream under capture runs the worst case.
+        uint32_t check = eager ? still : iters;
         bool live[4] = {true, true, true, true};
         for (uint32_t it = 0; it < iters; ++it) {
             if (it == check) {
+                if (it == still) {
+                    bool any = false;
+                    for (int h = 0; h < np; ++h) {
+                        GK_HIP(hipEventSynchronize(c.moved_ev[h]));
+                        live[h] = __atomic_load_n(c.h_word + h, __ATOMIC_RELAXED) != 0u;
+                        any = any || live[h];
+                    }
+                    if (!any) break;
+                }
                 for (int h = 0; h < np; ++h)
                     if (live[h])
                         GK_HIP(hipMemcpyAsync(c.h_word + h, QH[h].cnt + 2 * cur, sizeof(uint32_t),

@@ -350,7 +350,7 @@ def test_ref_v2_two_pipelines_give_the_single_pipeline_frame():
     (64, 64, 1, 4, 10, 0, False), (61, 35, 3, 8, 8, 0, False), (32, 32, 2, 1, 1, 0, False),
     (64, 48, 2, 4, 6, gk.FRAME_FAST_GATHER, False), (40, 40, 1, 3, 5, 0, True), (640, 416, 1, 6, 8, 0, False),
     # twelve samples of which each may wait once for its last sun ray
-    (40, 40, 3, 2, 2, 0, True)])
+    (40, 40, 3, 2, 2, 0, True), (640, 416, 1, 3, 5, 0, True)])
 def test_ref_v2_sun_rays_match_oracle(W, H, samples, bounces, max_bounces, flags, moved):
     """REF_V2 frames lit by a sun through the Cornell box's open front: the
     sun rays of a vertex and of the pixel's end answer as the oracle's, the paths draw the same
