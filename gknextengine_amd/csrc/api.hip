@@ -345,6 +345,7 @@ int gk_create(const gk_device_desc* desc, gk_ctx** out) {
         return GK_ERR_HIP;
     }
     for (auto& e : c.ev) (void)hipEventCreateWithFlags(&e, hipEventDisableSystemFence);
+    if (c.stamps.resize(4) != hipSuccess) { gk_destroy(ctx); return GK_ERR_OOM; }
     // gk_trace_static's array on this GPU; a failure is reported by gk_trace_static itself
     (void)static_scratch_init(c.device);
     const int s = alloc_targets(c);
@@ -645,7 +646,7 @@ int gk_target_info(gk_ctx* ctx, int target, size_t* bytes, void** device_ptr) {
 
 // Statistics since the context was created: ray counts and the trace launches' times from
 // the slots' device words, and the stage times of
-// the last frame (events ev[0..6] of render_frame / post_process).
+// the last frame (Ctx::timed).
 int gk_get_stats(gk_ctx* ctx, gk_stats* out) {
     GK_CHECK_CTX_KEEP(ctx);
     if (!out) return GK_ERR_ARG;
@@ -653,12 +654,26 @@ int gk_get_stats(gk_ctx* ctx, gk_stats* out) {
     GK_HIP(hipStreamSynchronize(c.stream));
     const int s = collect_timing(c);
     if (s != GK_OK) return s;
-    if (c.frames_rendered > 0) {
+    if (c.frames_rendered > 0 && c.timed != Ctx::Timed::none) {
         float a = 0.f, b = 0.f, r = 0.f, d = 0.f;
-        if (hipEventElapsedTime(&a, c.ev[0], c.ev[1]) == hipSuccess) c.stats.ms_tlas = a;
-        if (hipEventElapsedTime(&b, c.ev[0], c.ev[3]) == hipSuccess) c.stats.ms_frame = b;
-        if (hipEventElapsedTime(&r, c.ev[4], c.ev[5]) == hipSuccess) c.stats.ms_reproject = r;
-        if (hipEventElapsedTime(&d, c.ev[5], c.ev[6]) == hipSuccess) c.stats.ms_denoise = d;
+        if (!c.tlas_timed) c.stats.ms_tlas = 0.0;
+        else if (hipEventElapsedTime(&a, c.ev[0], c.ev[1]) == hipSuccess) c.stats.ms_tlas = a;
+        if (c.timed == Ctx::Timed::stamps) {
+            unsigned long long t[4];
+            int khz = 0;
+            GK_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, c.device));
+            GK_HIP(hipMemcpy(t, c.stamps.ptr, sizeof(t), hipMemcpyDeviceToHost));
+            auto ms = [&](int i, int j) { return t[j] > t[i] ? double(t[j] - t[i]) / double(std::max(khz, 1)) : 0.0; };
+            c.stats.ms_frame = c.stats.ms_tlas + ms(0, 3);
+            c.stats.ms_reproject = ms(1, 2);
+            c.stats.ms_denoise = ms(2, 3);
+        } else {
+            if (hipEventElapsedTime(&b, c.ev[0], c.ev[3]) == hipSuccess) c.stats.ms_frame = b;
+            if (c.timed == Ctx::Timed::events) {
+                if (hipEventElapsedTime(&r, c.ev[4], c.ev[5]) == hipSuccess) c.stats.ms_reproject = r;
+                if (hipEventElapsedTime(&d, c.ev[5], c.ev[6]) == hipSuccess) c.stats.ms_denoise = d;
+            }
+        }
     }
     c.stats.extension_rays = c.stats.rays_traced - c.stats.shadow_rays;
     *out = c.stats;

@@ -300,7 +300,14 @@ struct Ctx {
         DevBuf<uint32_t> pspill[3];           // the same for trace slots 1..3
     } wf;
 
-    // stage times of the last frame; like the fork and join events without a system-scope fence
+    // Stage times of the last frame. Frames with the bilateral post passes: clock stamps by the
+    // kernels themselves (start of the frame, of k_reproject and of k_jbf, end of k_jbf); each
+    // event in their place costs 4 to 5 us (16 preview frames at 256x256 with seven each, and a
+    // history copy now part of k_jbf: 3.00 -> 2.64 ms). Others, and a TLAS update: events.
+    enum class Timed { none, stamps, events, events_no_post } timed = Timed::none;
+    bool tlas_timed = false;
+    DevBuf<unsigned long long> stamps;
+    // events: like the fork and join events without a system-scope fence
     // (only this device's streams and its clock use them, and a fence writes every L2 back):
     // the preview above 3.47 -> 3.32 ms, the city frames 10.9 -> 10.7 ms
     hipEvent_t ev[16] = {};

@@ -1177,8 +1177,10 @@ __global__ void k_pt_finalize(FrameK K, Targets T, PathState S, uint32_t n, uint
     }
 }
 
-__global__ void k_copy_objid(const uint32_t* a, uint32_t* b, uint32_t n) {
+// stamp (may be null): the frame's start
+__global__ void k_copy_objid(const uint32_t* a, uint32_t* b, uint32_t n, unsigned long long* stamp) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0u && stamp) *stamp = wall_clock64();
     if (i < n) b[i] = a[i];
 }
 
@@ -1271,10 +1273,13 @@ int render_frame(Ctx& c) {
     auto& w = c.wf;
     hipStream_t s = c.stream;
     const uint32_t n = c.width * c.height;
-    hipEventRecord(c.ev[0], s);
-    if (c.params.flags & GK_FRAME_POST_ONLY) {  // the caller wrote the rt pass's targets
-        hipEventRecord(c.ev[1], s);
-        hipEventRecord(c.ev[2], s);
+    const bool post_only = c.params.flags & GK_FRAME_POST_ONLY, skip_post = c.params.flags & GK_FRAME_SKIP_POST;
+    const bool stamped = !post_only && !skip_post && c.params.denoiser != GK_DENOISER_UNET;
+    c.timed = stamped ? Ctx::Timed::stamps
+                      : (skip_post && !post_only ? Ctx::Timed::events_no_post : Ctx::Timed::events);
+    c.tlas_timed = c.tlas_dirty && !post_only;
+    if (!stamped || c.tlas_timed) hipEventRecord(c.ev[0], s);
+    if (post_only) {  // the caller wrote the rt pass's targets
         st = post_process(c);
         if (st != GK_OK) return st;
         hipEventRecord(c.ev[3], s);
@@ -1285,7 +1290,7 @@ int render_frame(Ctx& c) {
         st = (c.params.flags & GK_FRAME_TLAS_REBUILD) ? rebuild_tlas(c) : refit_tlas(c);
         if (st != GK_OK) return st;
     }
-    hipEventRecord(c.ev[1], s);
+    if (tlas_work) hipEventRecord(c.ev[1], s);
     const FrameK K = make_k(c);
     const DScene S0 = make_dscene(c);
     Targets T;
@@ -1332,7 +1337,8 @@ int render_frame(Ctx& c) {
     P.rng2 = w.q_rng[0].ptr;  // queue state of PT_MIS, free in REF_V2
 
     // previous object ids for reprojection (copy pass, PathTracingRenderer.cpp:160-216)
-    k_copy_objid<<<nblk(n), 256, 0, s>>>(T.objid, static_cast<uint32_t*>(c.target_ptr[GK_RT_OBJECTID_1]), n);
+    k_copy_objid<<<nblk(n), 256, 0, s>>>(T.objid, static_cast<uint32_t*>(c.target_ptr[GK_RT_OBJECTID_1]), n,
+                                        stamped ? c.stamps.ptr : nullptr);
     GK_HIP(hipGetLastError());
     const bool ref = c.params.estimator == GK_ESTIMATOR_REF_V2;
     // Frames of many paths run as kPathParts path pipelines (part h: the 8x8 tiles h mod
@@ -1560,12 +1566,11 @@ int render_frame(Ctx& c) {
             GK_HIP(hipStreamWaitEvent(s, c.join_ev[h], 0));
         }
     }
-    hipEventRecord(c.ev[2], s);
-    if (!(c.params.flags & GK_FRAME_SKIP_POST)) {
+    if (!skip_post) {
         st = post_process(c);
         if (st != GK_OK) return st;
     }
-    hipEventRecord(c.ev[3], s);
+    if (!stamped) hipEventRecord(c.ev[3], s);
     c.early_ok = split && cap0 == hipStreamCaptureStatusNone;
     c.early_w = c.width;
     c.early_h = c.height;

@@ -395,3 +395,37 @@ def test_ref_v2_sun_rays_match_oracle(W, H, samples, bounces, max_bounces, flags
         lit = o["diffuse"][..., :3].max(axis=2) > 1.0
         assert lit.mean() > 0.02  # the sun reaches the box
         assert ctx.stats().shadow_rays > W * H
+
+
+@pytest.mark.parametrize("flags,unet", [(0, False), (gk.FRAME_SKIP_POST, False), (gk.FRAME_POST_ONLY, False), (0, True)])
+def test_stage_times_of_a_frame(flags, unet):
+    """The stage times add up whichever way they are taken: clock stamps of the post kernels, or
+    events around the learned denoiser, skipped post passes, and post passes alone."""
+    W, H = 333, 217
+    s = gk.procgen_cornell()
+    with gk.Context(W, H) as ctx:
+        ctx.upload(s)
+        if unet:
+            net = gk.UNet.pretrained(ctx)  # kept: the context renders with it
+        for f in range(3):
+            p = cornell_params(W, H, frame=f)
+            if unet:
+                p.denoiser = gk.DENOISER_UNET
+            if f:
+                p.flags |= flags
+            if f == 2:
+                w = np.eye(4, dtype=np.float32)
+                w[0, 3] = 0.01
+                ctx.update_instances(w[None])  # a TLAS update
+            ctx.frame(p)
+            ctx.render()
+            ctx.sync()
+            st = ctx.stats()
+            print(f, st.ms_tlas, st.ms_frame, st.ms_reproject, st.ms_denoise, flush=True)
+            assert 0.0 < st.ms_frame < 1000.0
+            assert 0.0 <= st.ms_tlas < st.ms_frame
+            if not (f and flags & gk.FRAME_SKIP_POST):
+                assert st.ms_reproject > 0.0 and st.ms_denoise > 0.0
+                assert st.ms_reproject + st.ms_denoise <= st.ms_frame
+            if f == 2 and not flags & gk.FRAME_POST_ONLY:
+                assert st.ms_tlas > 0.0
