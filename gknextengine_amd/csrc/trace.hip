@@ -295,6 +295,20 @@ __device__ inline void quad_min_hit(float& t, float& u, float& v, uint32_t& prim
     if (ot < t || (ot == t && op < prim)) { t = ot; u = ou; v = ov; prim = op; }
 }
 
+// Quads of a wave that take rays. A wave lasts as long as its slowest ray and runs the node and
+// the leaf code in turn as soon as two of its quads differ, so few rays are spread over one wave
+// per SIMD (1024 on 256 CUs, the first work-groups of every grid): 300 random rays into the
+// 64 x 64-lot city, call to answer, 60.3 -> 50.7 us. Over all waves of the grid, up to four per
+// SIMD, launches of some ten thousand rays ran longer (16 preview frames at 256x256: 2.66 ->
+// 2.68 ms; three 1280x720 windows: 1.74 -> 1.75 ms).
+constexpr uint32_t kSpreadWaves = 1024;
+__device__ inline uint32_t quad_share(uint32_t count) {
+    const uint32_t waves = gridDim.x * (kBlock / 64u);
+    const uint32_t over = waves < kSpreadWaves ? waves : kSpreadWaves;
+    const uint32_t per = (count + over - 1u) / over;
+    return per < 16u ? per : 16u;
+}
+
 template <int MODE, bool TWO>
 __device__ void trace_quads(const Bvh4Node* __restrict__ blas, const TriRec* __restrict__ tris,
                             const Bvh4Node* __restrict__ tlas, const uint32_t* __restrict__ tlas_prims,
@@ -303,8 +317,11 @@ __device__ void trace_quads(const Bvh4Node* __restrict__ blas, const TriRec* __r
                             uint32_t (*stack)[kQuads], uint32_t* __restrict__ overflow_flag) {
     const uint32_t q = __lane_id() & 3u;
     const uint32_t qi = threadIdx.x >> 2;
-    const uint32_t nquads = gridDim.x * kQuads;
-    for (uint32_t r = blockIdx.x * kQuads + qi; r < count; r += nquads) {
+    const uint32_t share = quad_share(count);
+    if ((qi & 15u) >= share) return;
+    const uint32_t waves = gridDim.x * (kBlock / 64u);
+    const uint32_t gw = blockIdx.x * (kBlock / 64u) + (threadIdx.x >> 6);
+    for (uint32_t r = gw * share + (qi & 15u); r < count; r += waves * share) {
         const bool second = MODE == 2 && r >= c0;
         const uint32_t ri = second ? r - c0 : r;
         const bool any = MODE == 1 || second;
@@ -468,7 +485,7 @@ __global__ __launch_bounds__(kBlock) void k_trace(
     if (count <= (TWO ? kQuadRaysTwo : kQuadRays) * gridDim.x * kQuads) {
         trace_quads<MODE, TWO>(blas, tris, tlas, tlas_prims, inst, blas_root, j0, j1, c0, count,
                                reinterpret_cast<uint32_t (*)[kQuads]>(lds), overflow_flag);
-        if ((gtid & ~63u) / 4u < count) stamp_end();  // a wave without a ray says nothing
+        if ((gtid >> 6) * quad_share(count) < count) stamp_end();  // a wave without a ray says nothing
         return;
     }
     // rays a wave holds at once: its share of the launch. The launch holds more rays than the

@@ -387,3 +387,28 @@ def test_trace_time_adds_up_over_launches_and_slots(device):
         ctx.sync()
         t = 1e3 * (time.perf_counter() - t)
         assert 0.02 < ctx.stats().ms_trace - last < 2 * t  # two launches run at a time
+
+
+@pytest.mark.parametrize("any_hit", [False, True])
+@pytest.mark.parametrize("two_level", [False, True])
+def test_small_launches_at_the_edges_of_a_waves_share(device, two_level, any_hit):
+    """Few rays are spread over one wave per SIMD, 1 to 16 to a wave: at the edges of a wave's
+    share every ray gets the oracle's answer."""
+    if two_level:
+        s, half = scenes.Bricks().scene, 14.0
+    else:
+        s, half = gk.procgen_cornell(), 1.0
+    osc = po.OracleScene(s)
+    rays = scenes.random_rays(16400, -half, half, seed=11)
+    want, winst = osc.trace(rays)
+    hit = _u32(want[:, 3]) != 0xFFFFFFFF
+    assert 0.1 < hit.mean()
+    with gk.Context(32, 32) as ctx:
+        ctx.upload(s)
+        for n in (1, 2, 63, 300, 1023, 1024, 1025, 2048, 2049, 15360, 15361, 16384, 16385):
+            h, inst = gpu_trace(ctx, rays[:n], device, any_hit)
+            if any_hit:
+                assert np.array_equal(_u32(h[:, 3]) == 1, hit[:n]), n
+            else:
+                assert np.array_equal(_u32(h), _u32(want[:n])), n
+                assert np.array_equal(inst[hit[:n]], winst[:n][hit[:n]]), n
