@@ -652,7 +652,7 @@ __global__ __launch_bounds__(256) void k_ref_primary(DScene s, FrameK K, Targets
 // the random state kept in S.rng2 and the extension hit is dropped. A path that only waits for
 // its sun ray has an extension entry that traces nothing (null_ray).
 // (Traced inside this kernel by one thread each, with the stack in scratch, the sun rays took
-// most of it: 1080p city with sun, sky and probes 16.7 ms for four frames, 13.5 now, with the
+// most of it: 1080p city with sun, sky and probes 16.7 ms for four frames, 13.1 now, with the
 // probe lookup of gk_probe.hpp. In a queue that delayed their paths by a launch: 14.7 ms, twice
 // the launches, of which the last ten hold a few hundred paths and take as long as their
 // dependent loads, 25 to 80 us each. Four waves per SIMD instead of three spill: 14.0 ms.)
