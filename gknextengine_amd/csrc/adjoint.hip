@@ -51,6 +51,7 @@ struct DiffK {
     uint32_t W, H, frame0, seed, spp, bounces, has_sky;
     uint32_t tiles_x, tiles;  // 8 x 8 pixel tiles, the last ones of a row or column partly outside
     uint32_t streams;         // waves of a work-group on the same tile (1, 2 or 4)
+    uint32_t* overflow;       // SingleStack::overflow
 };
 
 // One scattering vertex of a path under differentiation, in planes of one entry per thread.
@@ -354,7 +355,7 @@ __global__ __launch_bounds__(256, TWO ? 3 : 4) void k_diff_primal(DScene s, Diff
     if (in)
         for (uint32_t smp = stream; smp < K.spp; smp += K.streams) {
             rng4 seed{x, y, K.frame0 + smp, K.seed};
-            acc = acc + dpath<false, TWO>(s, K, x, y, seed, (SingleStack)&stacks[0][threadIdx.x], f3{0, 0, 0}, nullptr, PathRec{}, 0u,
+            acc = acc + dpath<false, TWO>(s, K, x, y, seed, SingleStack{(SingleStack::Column)&stacks[0][threadIdx.x], K.overflow}, f3{0, 0, 0}, nullptr, PathRec{}, 0u,
                                            nrec);
         }
     __syncthreads();
@@ -392,7 +393,7 @@ __global__ __launch_bounds__(256, TWO ? 3 : 4) void k_diff_adjoint(DScene s, Dif
             for (uint32_t smp = stream; smp < K.spp; smp += K.streams) {
                 rng4 seed{x, y, K.frame0 + smp, K.seed};
                 uint32_t nrec = 0;
-                const f3 Ltot = dpath<true, TWO>(s, K, x, y, seed, (SingleStack)&stacks[0][threadIdx.x], dL, g, rec, gtid, nrec);
+                const f3 Ltot = dpath<true, TWO>(s, K, x, y, seed, SingleStack{(SingleStack::Column)&stacks[0][threadIdx.x], K.overflow}, dL, g, rec, gtid, nrec);
                 scatter_gradients(s, rec, gtid, nrec, Ltot, dL, g);
             }
         }
@@ -434,6 +435,7 @@ DiffK make_diffk(const Ctx& c) {
     K.has_sky = c.params.has_sky;
     K.tiles_x = (K.W + 7u) / 8u;
     K.tiles = K.tiles_x * ((K.H + 7u) / 8u);
+    K.overflow = &c.words.ptr->single_overflow;
     K.streams = K.spp >= 4u ? 4u : (K.spp >= 2u ? 2u : 1u);
     return K;
 }

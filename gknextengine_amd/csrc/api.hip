@@ -345,7 +345,9 @@ int gk_create(const gk_device_desc* desc, gk_ctx** out) {
         return GK_ERR_HIP;
     }
     for (auto& e : c.ev) (void)hipEventCreateWithFlags(&e, hipEventDisableSystemFence);
-    if (c.stamps.resize(4) != hipSuccess) { gk_destroy(ctx); return GK_ERR_OOM; }
+    if (c.words.resize(1) != hipSuccess) { gk_destroy(ctx); return GK_ERR_OOM; }
+    constexpr size_t w16 = sizeof(CtxWords) / 2;
+    k_fill_u16<<<uint32_t((w16 + 255) / 256), 256, 0, c.stream>>>(reinterpret_cast<uint16_t*>(c.words.ptr), w16, 0);
     // gk_trace_static's array on this GPU; a failure is reported by gk_trace_static itself
     (void)static_scratch_init(c.device);
     const int s = alloc_targets(c);
@@ -654,15 +656,21 @@ int gk_get_stats(gk_ctx* ctx, gk_stats* out) {
     GK_HIP(hipStreamSynchronize(c.stream));
     const int s = collect_timing(c);
     if (s != GK_OK) return s;
+    CtxWords words;
+    GK_HIP(hipMemcpy(&words, c.words.ptr, sizeof(words), hipMemcpyDeviceToHost));
+    if (words.single_overflow) {  // reported below; the device flag starts over
+        c.stack_overflow = true;
+        const uint32_t zero = 0;
+        GK_HIP(hipMemcpy(&c.words.ptr->single_overflow, &zero, 4, hipMemcpyHostToDevice));
+    }
     if (c.frames_rendered > 0 && c.timed != Ctx::Timed::none) {
         float a = 0.f, b = 0.f, r = 0.f, d = 0.f;
         if (!c.tlas_timed) c.stats.ms_tlas = 0.0;
         else if (hipEventElapsedTime(&a, c.ev[0], c.ev[1]) == hipSuccess) c.stats.ms_tlas = a;
         if (c.timed == Ctx::Timed::stamps) {
-            unsigned long long t[4];
+            const unsigned long long* t = words.stamp;
             int khz = 0;
             GK_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, c.device));
-            GK_HIP(hipMemcpy(t, c.stamps.ptr, sizeof(t), hipMemcpyDeviceToHost));
             auto ms = [&](int i, int j) { return t[j] > t[i] ? double(t[j] - t[i]) / double(std::max(khz, 1)) : 0.0; };
             c.stats.ms_frame = c.stats.ms_tlas + ms(0, 3);
             c.stats.ms_reproject = ms(1, 2);
@@ -680,8 +688,9 @@ int gk_get_stats(gk_ctx* ctx, gk_stats* out) {
     bool static_ovf = false;
     const int so = static_scratch_overflow(c, static_ovf);
     if (so != GK_OK) return so;
-    // a traversal stack overflowed since the last report (gk_trace, gk_render, or the last
-    // gk_trace_static on this GPU): those results are invalid; reported once
+    // a traversal stack overflowed since the last report (gk_trace, gk_render,
+    // gk_render_radiance, gk_adjoint, or the last gk_trace_static on this GPU): those results
+    // are invalid; reported once
     const bool ovf = c.stack_overflow || static_ovf;
     c.stack_overflow = false;
     return ovf ? GK_ERR_LIMIT : GK_OK;

@@ -167,6 +167,13 @@ __device__ inline void trace_slot_next(TraceSlot* s) {
     }
 }
 
+// Device words of a context that gk_get_stats reads.
+struct CtxWords {
+    unsigned long long stamp[4];  // clock stamps of the last frame (Ctx::Timed::stamps)
+    uint32_t single_overflow;     // a stack of the differentiable renderer's traversal overflowed
+    uint32_t pad;
+};
+
 // ------------------------------------------------------------------ context
 struct Ctx {
     int device = 0;
@@ -306,7 +313,7 @@ struct Ctx {
     // history copy now part of k_jbf: 3.00 -> 2.64 ms). Others, and a TLAS update: events.
     enum class Timed { none, stamps, events, events_no_post } timed = Timed::none;
     bool tlas_timed = false;
-    DevBuf<unsigned long long> stamps;
+    DevBuf<CtxWords> words;             // one, zeroed by gk_create
     // events: like the fork and join events without a system-scope fence
     // (only this device's streams and its clock use them, and a fence writes every L2 back):
     // the preview above 3.47 -> 3.32 ms, the city frames 10.9 -> 10.7 ms

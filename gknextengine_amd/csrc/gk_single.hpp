@@ -7,20 +7,29 @@
 // far with the internal ones, and in single-level scenes a lane keeps the leaf it reaches and
 // goes on with nodes, and the wave tests leaves together once half of its live lanes hold one
 // (leaves tested as they are met run the triangle code for a few lanes at a time). The stack's
-// first kSingleLds entries are a column per thread in LDS, deeper ones private memory.
+// first kSingleLds entries are a column per thread in LDS, deeper ones private memory; a ray
+// that needs more of them ends, and says so.
 #pragma once
 #include "gk_scene.hpp"
 
 namespace gk {
 
 constexpr uint32_t kSingleLds = 24;    // stack entries per thread in LDS
-constexpr uint32_t kSingleDeep = 72;   // further entries in private memory
+// Further entries in private memory. Geometry in nested clusters makes a radix tree of 63-bit
+// codes a chain; its wide nodes take three binary levels each and leave three waiting entries
+// on each of about 30 levels, in both levels of the scene, with a mark between them. (Leaves
+// wait as entries; tested as they are met they took none, and 96 held such a scene.)
+constexpr uint32_t kSingleDeep = 168;
 constexpr uint32_t kSingleNone = 0xfffffffeu;
 
-// This thread's column of the LDS part, entry k at [k * blockDim.x]. A pointer of the LDS
-// address space: with a generic one the compiler turns a pop, which reads LDS or private
-// memory, into one flat load of a chosen address.
-typedef __attribute__((address_space(3))) uint32_t* SingleStack;
+struct SingleStack {
+    // This thread's column of the LDS part, entry k at [k * blockDim.x]. A pointer of the LDS
+    // address space: with a generic one the compiler turns a pop, which reads LDS or private
+    // memory, into one flat load of a chosen address.
+    typedef __attribute__((address_space(3))) uint32_t* Column;
+    Column lds;
+    uint32_t* overflow;  // set to 1 when a ray ended because its stack was full
+};
 
 template <bool ANY, bool TWO>
 __device__ inline bool trace_single(const DScene& s, const f3 wO, const f3 wD, const float tmin, const float tmax,
@@ -28,16 +37,19 @@ __device__ inline bool trace_single(const DScene& s, const f3 wO, const f3 wD, c
     uint32_t deep[kSingleDeep];
     uint32_t sp = 0;
     const uint32_t stride = blockDim.x;
+    // An entry past the last one is counted but not kept, and the ray ends with the step that
+    // pushed it. (The return mark of an instance always fits: it takes the place of the
+    // instance's entry, popped just before.)
+    constexpr uint32_t kFull = kSingleLds + kSingleDeep;
     auto push = [&](uint32_t e) {
-        if (sp < kSingleLds) stack[sp * stride] = e;
-        else if (sp < kSingleLds + kSingleDeep) deep[sp - kSingleLds] = e;
-        else return;
+        if (sp < kSingleLds) stack.lds[sp * stride] = e;
+        else if (sp < kFull) deep[sp - kSingleLds] = e;
         ++sp;
     };
     auto pop = [&]() {
         --sp;
         uint32_t e;
-        if (sp < kSingleLds) e = stack[sp * stride];
+        if (sp < kSingleLds) e = stack.lds[sp * stride];
         else e = deep[sp - kSingleLds];
         return e;
     };
@@ -208,8 +220,10 @@ __device__ inline bool trace_single(const DScene& s, const f3 wO, const f3 wD, c
                 if (TWO && (kc[0] & kInstFlag)) push(kc[0]);  // instances are entered by the pop path
                 else node = kc[0];
             }
+            if (sp > kFull) active = false;
         }
     }
+    if (sp > kFull) atomicOr(stack.overflow, 1u);
     return found;
 }
 

@@ -40,7 +40,7 @@ struct PostT {
     const uint16_t* moment;
     ushort4* out;
     ushort4 *hist_d, *hist_s, *hist_a;    // k_jbf: the next frame's prev_*
-    unsigned long long* stamp;            // clock stamps (may be null): Ctx::stamps
+    unsigned long long* stamp;            // clock stamps (may be null): CtxWords::stamp
 };
 
 // The previous frame's 2x2 footprint at (px, py), with px, py inside the image: element
@@ -361,7 +361,7 @@ int post_process(Ctx& c) {
     T.hist_s = prev_s;
     T.hist_a = prev_a;
     const bool events = c.timed != Ctx::Timed::stamps;
-    T.stamp = events ? nullptr : c.stamps.ptr;
+    T.stamp = events ? nullptr : c.words.ptr->stamp;
     if (events) hipEventRecord(c.ev[4], c.stream);
     k_reproject<<<grid, blk, 0, c.stream>>>(K, T);
     GK_HIP(hipGetLastError());

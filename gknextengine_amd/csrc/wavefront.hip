@@ -1338,7 +1338,7 @@ int render_frame(Ctx& c) {
 
     // previous object ids for reprojection (copy pass, PathTracingRenderer.cpp:160-216)
     k_copy_objid<<<nblk(n), 256, 0, s>>>(T.objid, static_cast<uint32_t*>(c.target_ptr[GK_RT_OBJECTID_1]), n,
-                                        stamped ? c.stamps.ptr : nullptr);
+                                        stamped ? c.words.ptr->stamp : nullptr);
     GK_HIP(hipGetLastError());
     const bool ref = c.params.estimator == GK_ESTIMATOR_REF_V2;
     // Frames of many paths run as kPathParts path pipelines (part h: the 8x8 tiles h mod

@@ -432,8 +432,9 @@ int gk_write_target(gk_ctx* ctx, int target, const void* host, size_t bytes);
 int gk_target_info(gk_ctx* ctx, int target, size_t* bytes, void** device_ptr);
 
 /* Statistics since the context was created. GK_ERR_LIMIT (with *out filled) when a
- * traversal stack overflowed since the last call (gk_trace, gk_render, or the last
- * gk_trace_static on the context's GPU): those hits are invalid. Reported once. */
+ * traversal stack overflowed since the last call (gk_trace, gk_render, gk_render_radiance,
+ * gk_adjoint, or the last gk_trace_static on the context's GPU): those results are invalid.
+ * Reported once. */
 int gk_get_stats(gk_ctx* ctx, gk_stats* out);
 
 /* ---------------------------------------------------------------- ray casting */

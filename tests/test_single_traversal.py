@@ -1,0 +1,51 @@
+"""The one-ray-per-thread traversal of the differentiable renderer, compiled for the CPU from
+its own header (a wave of one lane, AddressSanitizer on): hits against a test of every
+triangle, chains of nodes whose waiting children fill the stack in both levels of a scene, and
+trees too deep for it, which must end the ray and say so."""
+from __future__ import annotations
+
+import shutil
+import subprocess
+from pathlib import Path
+
+import pytest
+
+HERE = Path(__file__).resolve().parent / "traversal"
+CSRC = HERE.parents[1] / "gknextengine_amd" / "csrc"
+
+
+@pytest.fixture(scope="module")
+def driver(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("needs g++")
+    d = tmp_path_factory.mktemp("traversal")
+    # beside the stand-in for gk_scene.hpp, which a quoted include finds first
+    for f in (HERE / "gk_scene.hpp", CSRC / "gk_single.hpp", CSRC / "gk_math.hpp"):
+        shutil.copy(f, d)
+    exe = d / "driver"
+    r = subprocess.run(["g++", "-O1", "-g", "-std=c++17", "-ffp-contract=off", "-Wno-attributes", "-fsanitize=address",
+                        f"-I{d}", f"-I{HERE}", str(HERE / "single_driver.cpp"), "-o", str(exe)],
+                       capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-3000:]
+    return exe
+
+
+def run(driver, *args):
+    r = subprocess.run([str(driver), *map(str, args)], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-2000:]
+
+
+def test_hits_match_a_test_of_every_triangle(driver):
+    run(driver, "random")
+
+
+# 30 wide levels: the longest chain that a binary radix tree of 63-bit codes makes (three binary
+# levels each, with the ties' bits)
+@pytest.mark.parametrize("top,levels", [(0, 30), (1, 30), (30, 1), (30, 30)])
+def test_chains_fit_the_stack(driver, top, levels):
+    run(driver, "chain", top, levels, 0)
+
+
+@pytest.mark.parametrize("top,levels", [(0, 80), (1, 80), (63, 4), (64, 4), (65, 4), (80, 80)])
+def test_a_full_stack_ends_the_ray(driver, top, levels):
+    run(driver, "chain", top, levels, 1)
