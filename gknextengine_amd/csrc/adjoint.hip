@@ -131,7 +131,7 @@ __device__ inline bool metal_live(const gk_material& m) { return m.material_mode
 
 // The path of one sample: its radiance. ADJ: also adds the next-event terms of dL * dC to g
 // and records the scattering vertices (rec, entry gtid of each plane, nrec of them).
-template <bool ADJ, bool TWO>
+template <bool ADJ, SingleScene SCENE>
 __device__ inline f3 dpath(const DScene& s, const DiffK& K, uint32_t x, uint32_t y, rng4& seed, SingleStack stack, f3 dL,
                            float* g /* LDS, 5 per material */, const PathRec& rec, uint32_t gtid, uint32_t& nrec) {
     f3 O, D;
@@ -145,7 +145,7 @@ __device__ inline f3 dpath(const DScene& s, const DiffK& K, uint32_t x, uint32_t
     auto add = [&](f3 C) { Lsum = Lsum + C; };
     for (uint32_t depth = 0;; ++depth) {
         SHit h;
-        if (!trace_single<false, TWO>(s, O, D, 0.f, 1e30f, h, stack)) {
+        if (!trace_single<false, SCENE>(s, O, D, 0.f, 1e30f, h, stack)) {
             if (K.has_sky) {
                 const float4 sky = sky_radiance(s, K.sky, K.sky_rot, D);
                 add(T * f3{sky.x, sky.y, sky.z});
@@ -231,7 +231,7 @@ __device__ inline f3 dpath(const DScene& s, const DiffK& K, uint32_t x, uint32_t
             if (cosl > 0.f && wil.z > 0.f && dot(Ng, wl) > 0.f && psel > 0.f) {
                 const float pl = psel * d2 / (cosl * L.p0.w);
                 SHit unused;
-                if (!trace_single<true, TWO>(s, Po, wl, 0.f, dist * (1.f - 1e-4f) - off, unused, stack)) {
+                if (!trace_single<true, SCENE>(s, Po, wl, 0.f, dist * (1.f - 1e-4f) - off, unused, stack)) {
                     f3 fd, fs;
                     float pdd, pds;
                     bsdf_eval(b, wo, wil, fd, fs, pdd, pds);
@@ -344,8 +344,8 @@ __device__ inline void scatter_gradients(const DScene& s, const PathRec& rec, ui
 // Four waves per SIMD in single-level scenes (126 registers; at 129, three waves, the primal
 // takes 1.21 ms against 1.04 and the adjoint 1.33 against 1.25), three in two-level ones, whose
 // instance handling would spill.
-template <bool TWO>
-__global__ __launch_bounds__(256, TWO ? 3 : 4) void k_diff_primal(DScene s, DiffK K, float4* __restrict__ img) {
+template <SingleScene SCENE>
+__global__ __launch_bounds__(256, SCENE == SingleScene::two ? 3 : 4) void k_diff_primal(DScene s, DiffK K, float4* __restrict__ img) {
     __shared__ uint32_t stacks[kSingleLds][256];
     float (*part)[256] = reinterpret_cast<float (*)[256]>(&stacks[0][0]);  // after the paths
     uint32_t x, y, nrec = 0;
@@ -355,7 +355,7 @@ __global__ __launch_bounds__(256, TWO ? 3 : 4) void k_diff_primal(DScene s, Diff
     if (in)
         for (uint32_t smp = stream; smp < K.spp; smp += K.streams) {
             rng4 seed{x, y, K.frame0 + smp, K.seed};
-            acc = acc + dpath<false, TWO>(s, K, x, y, seed, SingleStack{(SingleStack::Column)&stacks[0][threadIdx.x], K.overflow}, f3{0, 0, 0}, nullptr, PathRec{}, 0u,
+            acc = acc + dpath<false, SCENE>(s, K, x, y, seed, SingleStack{(SingleStack::Column)&stacks[0][threadIdx.x], K.overflow}, f3{0, 0, 0}, nullptr, PathRec{}, 0u,
                                            nrec);
         }
     __syncthreads();
@@ -374,8 +374,8 @@ __global__ __launch_bounds__(256, TWO ? 3 : 4) void k_diff_primal(DScene s, Diff
 
 // grad partials: one row of 5*nmat floats per work-group; groups: tile groups of the image,
 // which the work-groups of the launch take in turn
-template <bool TWO>
-__global__ __launch_bounds__(256, TWO ? 3 : 4) void k_diff_adjoint(DScene s, DiffK K, const float4* __restrict__ dimg, PathRec rec,
+template <SingleScene SCENE>
+__global__ __launch_bounds__(256, SCENE == SingleScene::two ? 3 : 4) void k_diff_adjoint(DScene s, DiffK K, const float4* __restrict__ dimg, PathRec rec,
                                                       float* __restrict__ partial, uint32_t nparam, uint32_t groups) {
     extern __shared__ float g[];
     __shared__ uint32_t stacks[kSingleLds][256];
@@ -393,7 +393,7 @@ __global__ __launch_bounds__(256, TWO ? 3 : 4) void k_diff_adjoint(DScene s, Dif
             for (uint32_t smp = stream; smp < K.spp; smp += K.streams) {
                 rng4 seed{x, y, K.frame0 + smp, K.seed};
                 uint32_t nrec = 0;
-                const f3 Ltot = dpath<true, TWO>(s, K, x, y, seed, SingleStack{(SingleStack::Column)&stacks[0][threadIdx.x], K.overflow}, dL, g, rec, gtid, nrec);
+                const f3 Ltot = dpath<true, SCENE>(s, K, x, y, seed, SingleStack{(SingleStack::Column)&stacks[0][threadIdx.x], K.overflow}, dL, g, rec, gtid, nrec);
                 scatter_gradients(s, rec, gtid, nrec, Ltot, dL, g);
             }
         }
@@ -467,7 +467,8 @@ int gk_render_radiance(gk_ctx* ctx, float* d_image) {
         if (st != GK_OK) return st;
     }
     const DiffK K = make_diffk(c);
-    auto* kern = c.blas_only ? k_diff_primal<false> : k_diff_primal<true>;
+    auto* kern = !c.blas_only ? k_diff_primal<SingleScene::two>
+               : c.bvh_stats.blas_nodes > kSingleNear ? k_diff_primal<SingleScene::far> : k_diff_primal<SingleScene::near>;
     kern<<<tile_groups(K), 256, 0, c.stream>>>(make_dscene(c), K, reinterpret_cast<float4*>(d_image));
     GK_HIP(hipGetLastError());
     return GK_OK;
@@ -502,7 +503,8 @@ int gk_adjoint(gk_ctx* ctx, const float* d_dl_dimage, float* d_grad) {
     rec.b = rec.a + plane * verts;
     rec.c = reinterpret_cast<float*>(rec.b + plane * verts);
     rec.plane = uint32_t(plane);
-    auto* kern = c.blas_only ? k_diff_adjoint<false> : k_diff_adjoint<true>;
+    auto* kern = !c.blas_only ? k_diff_adjoint<SingleScene::two>
+               : c.bvh_stats.blas_nodes > kSingleNear ? k_diff_adjoint<SingleScene::far> : k_diff_adjoint<SingleScene::near>;
     // gradients (dynamic) and traversal stacks (static) above the default 64 KB of LDS
     if (nparam * 4u + kSingleLds * 1024u > 65536u)
         GK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,

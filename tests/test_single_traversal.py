@@ -49,3 +49,10 @@ def test_chains_fit_the_stack(driver, top, levels):
 @pytest.mark.parametrize("top,levels", [(0, 80), (1, 80), (63, 4), (64, 4), (65, 4), (80, 80)])
 def test_a_full_stack_ends_the_ray(driver, top, levels):
     run(driver, "chain", top, levels, 1)
+
+
+# the last nodes of a scene that 32 bits of offset reach, the first beyond, the most a scene of
+# 2^27 triangles can hold
+@pytest.mark.parametrize("at", [1, (1 << 25) - 2, (1 << 25) - 1, 1 << 25, (1 << 27) - 2])
+def test_nodes_past_4_gib(driver, at):
+    run(driver, "far", at)

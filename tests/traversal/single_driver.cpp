@@ -7,6 +7,8 @@
 #include <string>
 #include <vector>
 
+#include <sys/mman.h>
+
 #include "gk_single.hpp"
 
 using namespace gk;
@@ -44,11 +46,11 @@ struct Run {
     SHit hit;
     uint32_t overflow;
 };
-template <bool ANY, bool TWO>
+template <bool ANY, SingleScene SCENE>
 Run trace(const DScene& s, f3 O, f3 D) {
     std::vector<uint32_t> lds(kSingleLds);  // exactly the entries a thread has
     Run r{};
-    r.found = trace_single<ANY, TWO>(s, O, D, 0.f, 1e30f, r.hit, SingleStack{lds.data(), &r.overflow});
+    r.found = trace_single<ANY, SCENE>(s, O, D, 0.f, 1e30f, r.hit, SingleStack{lds.data(), &r.overflow});
     return r;
 }
 
@@ -113,12 +115,14 @@ int random_scenes() {
                     const float d = f * dot(e2, q);
                     if (d > 0 && d < bt[two]) { bt[two] = d; bp[two] = __float_as_uint(t.v0.w); bi[two] = ii; }
                 }
-        const Run one = trace<false, false>(s, O, D), two = trace<false, true>(s, O, D);
-        const Run any = trace<true, false>(s, O, D), any2 = trace<true, true>(s, O, D);
+        const Run one = trace<false, SingleScene::near>(s, O, D), two = trace<false, SingleScene::two>(s, O, D);
+        const Run any = trace<true, SingleScene::near>(s, O, D), any2 = trace<true, SingleScene::two>(s, O, D);
         hits += one.found + two.found;
         bad += one.hit.prim != bp[0] || two.hit.prim != bp[1] || two.hit.inst != bi[1];
         bad += (one.found && one.hit.t != bt[0]) || (two.found && two.hit.t != bt[1]);
         bad += any.found != one.found || any2.found != two.found;
+        const Run far = trace<false, SingleScene::far>(s, O, D);
+        bad += far.found != one.found || far.hit.t != one.hit.t || far.hit.prim != one.hit.prim;
         bad += one.overflow | two.overflow | any.overflow | any2.overflow;
     }
     printf("random: %d bad of %d hits\n", bad, hits);
@@ -176,13 +180,39 @@ int chains(uint32_t top_levels, uint32_t levels, bool want_overflow) {
         bad += !ok;
     };
     if (top_levels == 0) {
-        check("closest, one level", trace<false, false>(s, O, D), true);
-        check("any, one level", trace<true, false>(s, O, D), false);
+        check("closest, one level", trace<false, SingleScene::near>(s, O, D), true);
+        check("closest, one level, far", trace<false, SingleScene::far>(s, O, D), true);
+        check("any, one level", trace<true, SingleScene::near>(s, O, D), false);
     } else {
-        check("closest, two levels", trace<false, true>(s, O, D), true);
-        check("any, two levels", trace<true, true>(s, O, D), false);
+        check("closest, two levels", trace<false, SingleScene::two>(s, O, D), true);
+        check("any, two levels", trace<true, SingleScene::two>(s, O, D), false);
     }
     return bad;
+}
+
+// A root at node `at` of an array that is reserved but not filled, with two leaves: the hit
+// lies in a node whose offset passes 32 bits when `at` is 2^25 - 1 or more.
+template <SingleScene SCENE>
+int far_node(uint32_t at) {
+    const size_t bytes = (size_t(at) + 2u) * sizeof(Bvh4Node);
+    void* mem = mmap(nullptr, bytes, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
+    if (mem == MAP_FAILED) return 1;
+    Bvh4Node* nodes = static_cast<Bvh4Node*>(mem);
+    const Box all{f3{1.f, -kBig, -kBig}, f3{kBig, kBig, kBig}};
+    nodes[at] = nodes[at + 1u] = empty_node();
+    set_child(nodes[at], 0, all, at + 1u, 0u);
+    set_child(nodes[at + 1u], 2, all, tri_leaf(0u, 2u), 2u);
+    const std::vector<TriRec> tris = chain_tris();
+    const uint32_t prims[1] = {0};
+    const InstDev inst[1] = {moved(f3{0.f, 0.f, 0.f}, at)};
+    Bvh4Node top = empty_node();
+    set_child(top, 0, all, 0u, 1u);
+    const DScene s{nodes, tris.data(), &top, prims, inst, at};
+    const Run r = trace<false, SCENE>(s, f3{0.f, 0.f, 0.f}, f3{1.f, 0.f, 0.f});
+    const bool ok = r.found && r.hit.t == 20.f && r.hit.prim == 7u;
+    printf("node %u: found %d %s\n", at, int(r.found), ok ? "ok" : "WRONG");
+    munmap(mem, bytes);
+    return !ok;
 }
 
 }  // namespace
@@ -192,5 +222,11 @@ int main(int argc, char** argv) {
     if (what == "random") return random_scenes();
     if (what == "chain" && argc == 5)
         return chains(uint32_t(atoi(argv[2])), uint32_t(atoi(argv[3])), atoi(argv[4]) != 0);
+    if (what == "far" && argc == 3) {
+        const uint32_t at = uint32_t(atoll(argv[2]));
+        int bad = far_node<SingleScene::far>(at) + far_node<SingleScene::two>(at);
+        if (uint64_t(at) + 2u <= kSingleNear) bad += far_node<SingleScene::near>(at);
+        return bad;
+    }
     return 2;
 }
