@@ -34,6 +34,7 @@
 //     edges; 2^-20 missed one such shared-edge hit, and the result depended on ray order).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "gk_ctx.hpp"
@@ -195,10 +196,13 @@ __device__ inline void near_far_offsets(Lane& L) {
 // (far - O) * rD are the min and the max of the two plane distances, bit for bit (the
 // rounded difference and the product by a nonzero reciprocal are monotonic, and no term
 // is NaN), so the entry is max3 of the near terms and the exit min3 of the far terms and
-// the per-axis min/max pairs of slab1 go away. nb: the node array; node: its index.
-__device__ inline void slab4_ordered(const char* __restrict__ nb, uint32_t node, const Lane& L, float limit,
+// the per-axis min/max pairs of slab1 go away. nb: the node array; node: its index. A node is
+// 32 bits of offset from the array, or, FAR, an address of 64 bits (kNearNodes).
+template <bool FAR>
+__device__ inline void slab4_ordered(const Bvh4Node* __restrict__ nodes, uint32_t node, const Lane& L, float limit,
                                      float tl[4], uint4& child, uint4& meta) {
-    const uint32_t base = node * uint32_t(sizeof(Bvh4Node));
+    const char* nb = reinterpret_cast<const char*>(nodes + (FAR ? node : 0u));
+    const uint32_t base = FAR ? 0u : node * uint32_t(sizeof(Bvh4Node));
     const uint32_t ax = base | L.sx, ay = base | L.sy, az = base | L.sz;
     auto ld = [&](uint32_t off) { return *reinterpret_cast<const float4*>(nb + off); };
     const float4 nx = ld(ax), fx = ld(ax ^ 16u);
@@ -452,7 +456,7 @@ __device__ void trace_quads(const Bvh4Node* __restrict__ blas, const TriRec* __r
     }
 }
 
-template <int MODE, bool TWO>
+template <int MODE, bool TWO, bool FAR>
 __global__ __launch_bounds__(kBlock) void k_trace(
     const Bvh4Node* __restrict__ blas, const TriRec* __restrict__ tris,
     const Bvh4Node* __restrict__ tlas, const uint32_t* __restrict__ tlas_prims,
@@ -668,7 +672,7 @@ __global__ __launch_bounds__(kBlock) void k_trace(
         const bool tl_level = TWO && L.level == 0;
         float tl[4];
         uint4 nch, nmeta;
-        slab4_ordered(reinterpret_cast<const char*>(tl_level ? tlas : blas), L.node, L, L.bt, tl, nch, nmeta);
+        slab4_ordered<FAR>(tl_level ? tlas : blas, L.node, L, L.bt, tl, nch, nmeta);
         const uint32_t ch[4] = {nch.x, nch.y, nch.z, nch.w};
         const uint32_t mt4[4] = {nmeta.x, nmeta.y, nmeta.z, nmeta.w};
         // TLAS leaves push their instances; BLAS leaves join the internal children as
@@ -768,6 +772,23 @@ TraceSlot* trace_slot(Ctx& c, int slot) {
     return reinterpret_cast<TraceSlot*>(sp.ptr + words);
 }
 
+// Nodes that 32 bits of offset reach (4 GiB). Scenes of more, in either level, take kernels
+// that form 64-bit addresses instead.
+constexpr size_t kNearNodes = size_t(1) << 25;
+
+using TraceKernel = void (*)(const Bvh4Node*, const TriRec*, const Bvh4Node*, const uint32_t*, const InstDev*, uint32_t,
+                             TraceJob, TraceJob, TraceSlot*, uint32_t*);
+template <bool TWO, bool FAR>
+static TraceKernel trace_kernel(int mode) {
+    return mode == 0 ? k_trace<0, TWO, FAR> : mode == 1 ? k_trace<1, TWO, FAR> : k_trace<2, TWO, FAR>;
+}
+// the kernel of a mode (as k_trace) for the context's scene; a TLAS has fewer nodes than instances
+static TraceKernel trace_kernel(const Ctx& c, int mode) {
+    const bool far = std::max<size_t>(c.bvh_stats.blas_nodes, c.h_instances.size()) > kNearNodes;
+    if (c.blas_only) return far ? trace_kernel<false, true>(mode) : trace_kernel<false, false>(mode);
+    return far ? trace_kernel<true, true>(mode) : trace_kernel<true, false>(mode);
+}
+
 // Launches one persistent trace over up to two jobs (mode as k_trace) in a slot (its stream
 // and spill area).
 static int launch_jobs(Ctx& c, int mode, const TraceJob& j0, const TraceJob& j1, int slot) {
@@ -778,11 +799,8 @@ static int launch_jobs(Ctx& c, int mode, const TraceJob& j0, const TraceJob& j1,
     hipStream_t st = slot ? c.pstream[slot - 1] : c.stream;
     uint32_t* spill = slot ? c.wf.pspill[slot - 1].ptr : c.wf.spill.ptr;
     if (!ready) k_slot_next<<<1, 64, 0, st>>>(ts);
-    const bool two = !c.blas_only;
     const uint32_t root = c.h_meshes.empty() ? 0u : c.h_meshes[0].root;
-    auto* kern = mode == 0 ? (two ? k_trace<0, true> : k_trace<0, false>)
-               : mode == 1 ? (two ? k_trace<1, true> : k_trace<1, false>)
-                           : (two ? k_trace<2, true> : k_trace<2, false>);
+    const TraceKernel kern = trace_kernel(c, mode);
     const uint32_t blocks = persistent_blocks(c.device, kern, c.trace_split ? kSplitBlocksPerCU : kMaxBlocksPerCU);
     kern<<<blocks, kBlock, 0, st>>>(c.blas_nodes.ptr, c.tris.ptr, c.tlas_nodes.ptr, c.tlas_prims.ptr, c.inst.ptr, root,
                                    j0, j1, ts, spill);
@@ -954,9 +972,8 @@ extern "C" int gk_trace_static(gk_ctx* ctx, const gk_ray* d_rays, uint32_t n, gk
     // the previous call's counters are still there: start from zero
     k_clear_words<<<1, 64, 0, c.stream>>>(base, 32u);
     const bool any = (flags & GK_TRACE_ANY) != 0;
-    const bool two = !c.blas_only;
     const uint32_t root = c.h_meshes.empty() ? 0u : c.h_meshes[0].root;
-    auto* kern = any ? (two ? k_trace<1, true> : k_trace<1, false>) : (two ? k_trace<0, true> : k_trace<0, false>);
+    const TraceKernel kern = trace_kernel(c, any ? 1 : 0);
     uint32_t blocks = persistent_blocks(c.device, kern);
     if (blocks > kStaticBlocks) blocks = kStaticBlocks;
     TraceJob j0{reinterpret_cast<const float4*>(d_rays), reinterpret_cast<const float4*>(d_rays) + 1, nullptr, n,

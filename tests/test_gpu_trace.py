@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import gknextengine_amd as gk
+from gknextengine_amd import scenes as gk_scenes
 from oracle import pyoracle as po
 from tests import scenes
 from tests.test_oracle import _compare_hits, _u32
@@ -412,3 +413,71 @@ def test_small_launches_at_the_edges_of_a_waves_share(device, two_level, any_hit
             else:
                 assert np.array_equal(_u32(h), _u32(want[:n])), n
                 assert np.array_equal(inst[hit[:n]], winst[:n][hit[:n]]), n
+
+
+@pytest.fixture(scope="module")
+def large_lattice():
+    """8192 x 12288 small triangles in the plane z = 0, one per unit cell: 56 million nodes."""
+    W, H = 8192, 12288
+    pos = np.empty((H, W, 3, 3), np.float32)
+    for k, (dx, dy) in enumerate([(0.25, 0.25), (0.75, 0.25), (0.25, 0.75)]):
+        pos[:, :, k, 0] = np.arange(W, dtype=np.float32)[None, :] + dx
+        pos[:, :, k, 1] = np.arange(H, dtype=np.float32)[:, None] + dy
+        pos[:, :, k, 2] = 0
+    return W, H, pos
+
+
+def _lattice_scene(pos, instances):
+    s = gk.SceneData()
+    s.add_mesh(pos.reshape(-1, 3), np.arange(pos.size // 3, dtype=np.uint32).reshape(-1, 3))
+    s.materials = [gk_scenes.material((0.3, 0.6, 0.9))]
+    for x in instances:
+        w = np.eye(4, dtype=np.float32)
+        w[0, 3] = x
+        s.add_instance(0, world=w)
+    return s
+
+
+@pytest.mark.parametrize("instances", [(0.0,), (0.0, 8192.0)])
+def test_more_nodes_than_32_bits_of_offset_reach(device, large_lattice, instances):
+    """Hits in a scene whose nodes pass 4 GiB: few rays (four lanes each) and many, closest and
+    any, one level and two; and the path tracer and the differentiable render of its far corner
+    equal those of the corner alone, whose rays meet the same triangles."""
+    import torch
+    W, H, pos = large_lattice
+    corner = np.ascontiguousarray(pos[H - 96:, W - 96:])
+    cam = dict(eye=(W - 48.0, H - 48.0, 20.0), target=(W - 48.5, H - 48.25, 0.0))
+    p = gk.make_frame_params(cam["eye"], cam["target"], 64, 64, fov=60.0, up=(0.0, 1.0, 0.0))
+    p.estimator = gk.ESTIMATOR_PT_MIS
+    p.samples, p.bounces, p.max_bounces, p.has_sky = 2, 2, 2, 1
+    p.sky_color[:] = [0.5, 0.7, 1.0, 1.0]
+    images = []
+    for scene in (_lattice_scene(pos, instances), _lattice_scene(corner, instances)):
+        with gk.Context(64, 64) as ctx:
+            ctx.upload(scene)
+            ctx.frame(p)
+            ctx.render()
+            img = torch.empty((64, 64, 4), dtype=torch.float32, device=device)
+            gk.check(gk.lib().gk_render_radiance(ctx.h, img.data_ptr()), "gk_render_radiance")
+            ctx.sync()
+            images.append((ctx.read("RADIANCE"), img.cpu().numpy()))
+            ctx.stats()  # no traversal overflow
+            if scene.meshes[0]["positions"].shape[0] < pos.size // 3:
+                continue
+            assert ctx.bvh_stats().blas_nodes > 1 << 25
+            g = np.random.default_rng(1)
+            for m in (3000, 1000000):
+                cx, cy, at = g.integers(0, W, m), g.integers(0, H, m), g.integers(0, len(instances), m)
+                hit = g.random(m) < 0.7
+                r = np.zeros((m, 8), np.float32)
+                r[:, 0] = cx + np.where(hit, 0.375, 0.875) + np.float32(instances)[at]
+                r[:, 1], r[:, 2] = cy + np.where(hit, 0.375, 0.875), 1
+                r[:, 6], r[:, 7] = -1, 1e30
+                h, inst = gpu_trace(ctx, r, device)
+                assert np.array_equal(_u32(h[:, 3]), np.where(hit, cy * W + cx, 0xFFFFFFFF).astype(np.uint32))
+                assert np.all(h[hit, 0] == 1) and np.array_equal(inst[hit], at[hit])
+                h, _ = gpu_trace(ctx, r, device, any_hit=True)
+                assert np.array_equal(_u32(h[:, 3]), hit.astype(np.uint32))
+    for a, b in zip(*images):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+        assert 0.3 < a[..., 0].mean() / a[..., 3].mean() < 0.6
