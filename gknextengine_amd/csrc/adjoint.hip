@@ -440,8 +440,6 @@ DiffK make_diffk(const Ctx& c) {
     return K;
 }
 
-constexpr size_t kRecBytes = size_t(96) << 20;
-
 uint32_t tile_groups(const DiffK& K) {
     const uint32_t per = 4u / K.streams;
     return (K.tiles + per - 1u) / per;
@@ -490,14 +488,23 @@ int gk_adjoint(gk_ctx* ctx, const float* d_dl_dimage, float* d_grad) {
     const DiffK K = make_diffk(c);
     const uint32_t groups = tile_groups(K);
     // work-groups: as many as are resident (4 or 3 per CU), since each writes a row of
-    // gradients; fewer where the records of so many paths would pass kRecBytes (more than 10
-    // bounces) or the image has fewer tile groups
+    // gradients, or the image's tile groups. Their records hold every vertex a path may have,
+    // 9.4 MB per bounce (604 MB at 64); a path touches those it has. Where the memory is not
+    // there, fewer work-groups take the image in more turns. (512 x 512, 4 spp, records kept to
+    // 96 MB, which are 170 work-groups at 64 bounces: 24.3 ms in a closed box, 7.1 ms now; paths
+    // of one vertex 0.23 ms, 0.10 now, as at every other limit.)
     const uint32_t verts = std::max(1u, K.bounces);
-    const uint32_t resident = c.blas_only ? 1024u : 768u;
-    const uint32_t blocks = std::min(groups, std::min(resident, uint32_t(kRecBytes / (size_t(256) * verts * 36u))));
+    uint32_t blocks = std::min(groups, c.blas_only ? 1024u : 768u);
+    for (;; blocks = (blocks + 1u) / 2u) {
+        const size_t need = size_t(blocks) * 256u * verts * 9u;
+        if (c.path_rec.count >= need) break;
+        const hipError_t e = c.path_rec.resize(need);
+        if (e == hipSuccess) break;
+        if (e != hipErrorOutOfMemory || blocks == 1u) GK_HIP(e);
+        (void)hipGetLastError();
+    }
     const size_t plane = size_t(blocks) * 256u;
     if (c.grad_partial.count < size_t(blocks) * nparam) GK_HIP(c.grad_partial.resize(size_t(blocks) * nparam));
-    if (c.path_rec.count < plane * verts * 9u) GK_HIP(c.path_rec.resize(plane * verts * 9u));
     PathRec rec;
     rec.a = reinterpret_cast<float4*>(c.path_rec.ptr);
     rec.b = rec.a + plane * verts;

@@ -294,3 +294,85 @@ def test_material_count_up_to_the_limit(count):
     n = len(base)
     assert torch.all(grads[1][n:] == 0)
     assert torch.allclose(grads[1][:n], grads[0], rtol=1e-4, atol=2e-6 * float(grads[0].abs().max()))
+
+
+def _plain_gradient(ctx, scene, p, dL):
+    """The gradient of sum(image * dL) by gk_adjoint itself, on paths of p's own seed."""
+    import torch
+    g = torch.empty((len(scene.materials), 5), dtype=torch.float32, device="cuda")
+    ctx.frame(p)
+    torch.cuda.synchronize()
+    gk.check(gk.lib().gk_adjoint(ctx.h, dL.data_ptr(), g.data_ptr()), "gk_adjoint")
+    ctx.sync()
+    return g
+
+
+def test_time_does_not_depend_on_a_bounce_limit_no_path_reaches():
+    """Paths that end at their second vertex cost the same whatever the limit: the launch keeps
+    its work-groups. (Records kept to 96 MB gave 170 work-groups at 64 bounces, 2.3 times as long.)"""
+    import time
+
+    import torch
+    W = H = 512
+    scene = gk.SceneData()
+    scene.add_mesh([[-50, 0, -50], [50, 0, -50], [50, 0, 50], [-50, 0, 50]], [[0, 2, 1], [0, 3, 2]])
+    scene.materials = [scenes.material((0.4, 0.6, 0.8))]
+    scene.add_instance(0)
+    p = gk.make_frame_params((0, 3, -4), (0, 0, 0), W, H, fov=50.0)
+    p.estimator, p.samples, p.has_sky, p.total_frames = gk.ESTIMATOR_PT_MIS, 4, 1, 1
+    p.sky_color[:] = [0.5, 0.5, 0.5, 1.0]
+    dL = torch.ones((H, W, 4), dtype=torch.float32, device="cuda")
+    best, grads = {}, {}
+    with gk.Context(W, H) as ctx:
+        ctx.upload(scene)
+        for turn in range(6):
+            for b in (4, 64):
+                p.bounces = p.max_bounces = b
+                grads[b] = _plain_gradient(ctx, scene, p, dL)
+                g = torch.empty_like(grads[b])
+                t = time.perf_counter()
+                for _ in range(10):
+                    gk.check(gk.lib().gk_adjoint(ctx.h, dL.data_ptr(), g.data_ptr()), "gk_adjoint")
+                ctx.sync()
+                best[b] = min(best.get(b, 1e9), time.perf_counter() - t)
+    assert best[64] < 1.5 * best[4], best
+    assert float(grads[4].abs().max()) > 0
+    # (LDS float atomics: the order of a work-group's additions differs from run to run)
+    assert torch.allclose(grads[4], grads[64], rtol=1e-5)
+
+
+def test_records_that_do_not_fit_take_fewer_work_groups(tmp_path):
+    """With 250 MB of device memory the 604 MB of records of a 64-bounce gradient over 512 x 512
+    pixels do not fit: fewer work-groups take the image in turns, each using its records and its
+    sums for several tiles, and the gradient is the same. (A child process: the limit is read
+    once per process.)"""
+    import os
+    import subprocess
+    import sys
+    import textwrap
+    from pathlib import Path
+    code = textwrap.dedent("""
+        import sys
+        sys.path.insert(0, %r)
+        import numpy as np
+        import torch
+        import gknextengine_amd as gk
+        from tests.test_gpu_adjoint import _plain_gradient, setup
+        W = H = 512
+        scene, nmat, p = setup(W, H, spp=4, bounces=64)
+        dL = torch.from_numpy(np.random.default_rng(3).normal(size=(H, W, 4)).astype(np.float32)).cuda()
+        with gk.Context(W, H) as ctx:
+            ctx.upload(scene)
+            np.save(sys.argv[1], _plain_gradient(ctx, scene, p, dL).cpu().numpy())
+    """) % (str(Path(__file__).resolve().parents[1]),)
+    out = []
+    for name, limit in (("all", None), ("few", 250 * 1000 * 1000)):
+        env = dict(os.environ)
+        if limit:
+            env["GKNX_DEVICE_MEMORY_LIMIT"] = str(limit)
+        f = tmp_path / f"{name}.npy"
+        r = subprocess.run([sys.executable, "-c", code, str(f)], env=env, capture_output=True, text=True, timeout=100)
+        assert r.returncode == 0, r.stderr[-2000:]
+        out.append(np.load(f))
+    assert np.abs(out[0]).max() > 0
+    np.testing.assert_allclose(out[1], out[0], rtol=1e-4, atol=2e-6 * np.abs(out[0]).max())
