@@ -20,8 +20,8 @@
 // traversal of the scene.)
 //
 // Parameters per material (5 floats): albedo r, g, b, roughness (fuzziness), metallic.
-// Gradient contributions are summed per work-group in LDS and the per-group partials are
-// added in a fixed order by a second kernel.
+// Gradient contributions are summed per work-group in LDS, 256 pixels at a time; these sums are
+// added in double, to the work-group's row, and the rows in a fixed order by a second kernel.
 //
 // A wave traces the 8 x 8 pixels of a tile, one sample of each; the waves of a work-group
 // take different samples of the same tile (up to 4) or different tiles.
@@ -372,51 +372,57 @@ __global__ __launch_bounds__(256, SCENE == SingleScene::two ? 3 : 4) void k_diff
     img[size_t(y) * K.W + x] = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, 1.f);
 }
 
-// grad partials: one row of 5*nmat floats per work-group; groups: tile groups of the image,
-// which the work-groups of the launch take in turn
+// grad partials: one row of 5*nmat doubles per work-group. The work-groups of the launch take
+// the tile groups of the image in turn and add their FP32 sums to the row after every K.streams
+// of them, so that such a sum holds the paths of at most 256 pixels whatever the image's size.
 template <SingleScene SCENE>
 __global__ __launch_bounds__(256, SCENE == SingleScene::two ? 3 : 4) void k_diff_adjoint(DScene s, DiffK K, const float4* __restrict__ dimg, PathRec rec,
-                                                      float* __restrict__ partial, uint32_t nparam, uint32_t groups) {
+                                                      double* __restrict__ partial, uint32_t nparam, uint32_t groups) {
     extern __shared__ float g[];
     __shared__ uint32_t stacks[kSingleLds][256];
-    for (uint32_t k = threadIdx.x; k < nparam; k += blockDim.x) g[k] = 0.f;
-    __syncthreads();
     const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t stream = (threadIdx.x >> 6) % K.streams;
-    for (uint32_t group = blockIdx.x; group < groups; group += gridDim.x) {
-        uint32_t x, y;
-        if (!tile_pixel(K, group, x, y)) continue;
-        const float inv = 1.f / float(K.spp);
-        const float4 dl4 = dimg[size_t(y) * K.W + x];
-        const f3 dL = f3{dl4.x * inv, dl4.y * inv, dl4.z * inv};  // image = mean over samples
-        if (dL.x != 0.f || dL.y != 0.f || dL.z != 0.f) {
-            for (uint32_t smp = stream; smp < K.spp; smp += K.streams) {
-                rng4 seed{x, y, K.frame0 + smp, K.seed};
-                uint32_t nrec = 0;
-                const f3 Ltot = dpath<true, SCENE>(s, K, x, y, seed, SingleStack{(SingleStack::Column)&stacks[0][threadIdx.x], K.overflow}, dL, g, rec, gtid, nrec);
-                scatter_gradients(s, rec, gtid, nrec, Ltot, dL, g);
+    double* row = partial + size_t(blockIdx.x) * nparam;
+    for (uint32_t first = blockIdx.x; first < groups; first += K.streams * gridDim.x) {
+        for (uint32_t k = threadIdx.x; k < nparam; k += blockDim.x) g[k] = 0.f;
+        __syncthreads();
+        for (uint32_t q = 0; q < K.streams; ++q) {
+            const uint32_t group = first + q * gridDim.x;
+            uint32_t x, y;
+            if (group >= groups || !tile_pixel(K, group, x, y)) continue;
+            const float inv = 1.f / float(K.spp);
+            const float4 dl4 = dimg[size_t(y) * K.W + x];
+            const f3 dL = f3{dl4.x * inv, dl4.y * inv, dl4.z * inv};  // image = mean over samples
+            if (dL.x != 0.f || dL.y != 0.f || dL.z != 0.f) {
+                for (uint32_t smp = stream; smp < K.spp; smp += K.streams) {
+                    rng4 seed{x, y, K.frame0 + smp, K.seed};
+                    uint32_t nrec = 0;
+                    const f3 Ltot = dpath<true, SCENE>(s, K, x, y, seed, SingleStack{(SingleStack::Column)&stacks[0][threadIdx.x], K.overflow}, dL, g, rec, gtid, nrec);
+                    scatter_gradients(s, rec, gtid, nrec, Ltot, dL, g);
+                }
             }
         }
+        __syncthreads();
+        for (uint32_t k = threadIdx.x; k < nparam; k += blockDim.x)
+            row[k] = first == blockIdx.x ? double(g[k]) : row[k] + double(g[k]);
     }
-    __syncthreads();
-    float* row = partial + size_t(blockIdx.x) * nparam;
-    for (uint32_t k = threadIdx.x; k < nparam; k += blockDim.x) row[k] = g[k];
 }
 
-// 32 parameters per work-group, 8 threads of interleaved rows each, added in a fixed order
-// (1024 rows of 1285: 250 us with one thread per parameter over all rows, 40 us now)
-__global__ __launch_bounds__(256) void k_reduce_partials(const float* __restrict__ partial, uint32_t rows, uint32_t nparam,
+// 32 parameters per work-group, 32 threads of interleaved rows each, added in a fixed order
+// (1024 rows of 1285: 250 us with one thread per parameter over all rows, 40 us with 8 of FP32
+// rows, 12 us with 32)
+__global__ __launch_bounds__(1024) void k_reduce_partials(const double* __restrict__ partial, uint32_t rows, uint32_t nparam,
                                   float* __restrict__ out) {
-    __shared__ double red[8][32];
+    __shared__ double red[32][32];
     const uint32_t c = threadIdx.x & 31u, r0 = threadIdx.x >> 5;
     const uint32_t k = blockIdx.x * 32u + c;
     double acc = 0.0;
     if (k < nparam)
-        for (uint32_t r = r0; r < rows; r += 8u) acc += double(partial[size_t(r) * nparam + k]);
+        for (uint32_t r = r0; r < rows; r += 32u) acc += partial[size_t(r) * nparam + k];
     red[r0][c] = acc;
     __syncthreads();
     if (r0 != 0u || k >= nparam) return;
-    for (int q = 1; q < 8; ++q) acc += red[q][c];
+    for (int q = 1; q < 32; ++q) acc += red[q][c];
     out[k] = float(acc);
 }
 
@@ -519,7 +525,7 @@ int gk_adjoint(gk_ctx* ctx, const float* d_dl_dimage, float* d_grad) {
     kern<<<blocks, 256, nparam * 4, c.stream>>>(make_dscene(c), K, reinterpret_cast<const float4*>(d_dl_dimage), rec,
                                                 c.grad_partial.ptr, nparam, groups);
     GK_HIP(hipGetLastError());
-    k_reduce_partials<<<(nparam + 31) / 32, 256, 0, c.stream>>>(c.grad_partial.ptr, blocks, nparam, d_grad);
+    k_reduce_partials<<<(nparam + 31) / 32, 1024, 0, c.stream>>>(c.grad_partial.ptr, blocks, nparam, d_grad);
     GK_HIP(hipGetLastError());
     return GK_OK;
 }

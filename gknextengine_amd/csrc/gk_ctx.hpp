@@ -242,7 +242,7 @@ struct Ctx {
     DevBuf<float4> light_power;     // staging for gk_materials_update: per light (le rgb, pdf)
     BuildScratch scratch;
     gk_bvh_stats bvh_stats{};
-    DevBuf<float> grad_partial;     // adjoint: per-work-group gradient rows
+    DevBuf<double> grad_partial;    // adjoint: per-work-group gradient rows
     DevBuf<float> path_rec;         // adjoint: the scattering vertices of the paths in flight
     ::gk_unet* unet = nullptr;      // learned denoiser (GK_DENOISER_UNET), owned by the context
     std::vector<gk_light> h_lights; // LightObject quads (the probe bake lights with the first)

@@ -376,3 +376,41 @@ def test_records_that_do_not_fit_take_fewer_work_groups(tmp_path):
         out.append(np.load(f))
     assert np.abs(out[0]).max() > 0
     np.testing.assert_allclose(out[1], out[0], rtol=1e-4, atol=2e-6 * np.abs(out[0]).max())
+
+
+def test_sums_of_32_bits_hold_256_pixels():
+    """512 x 576 pixels at one sample are 1152 tile groups of 256 pixels on 1024 work-groups. A
+    pixel of group 0 weighs 2^20, one of group 1 cancels it, and the 64 of a tile of group 1024,
+    which the work-group of group 0 takes next and by the same wave, weigh 2^-6: added to the
+    first pixel's share in 32 bits each is below half of its last bit and is lost. (The order
+    within a wave's tile aside, nothing here depends on timing.)"""
+    import torch
+    W, H = 512, 576
+    scene = gk.SceneData()
+    scene.add_mesh([[-50, 0, -50], [50, 0, -50], [50, 0, 50], [-50, 0, 50]], [[0, 2, 1], [0, 3, 2]])
+    scene.materials = [scenes.material((0.5, 0.5, 0.5))]
+    scene.add_instance(0)
+    p = gk.make_frame_params((0, 3, -4), (0, 0, 0), W, H, fov=40.0)
+    p.estimator, p.samples, p.has_sky, p.total_frames = gk.ESTIMATOR_PT_MIS, 1, 1, 1
+    p.bounces = p.max_bounces = 2
+    p.sky_color[:] = [0.5, 0.5, 0.5, 1.0]
+    zero = torch.zeros((H, W, 4), dtype=torch.float32, device="cuda")
+    with gk.Context(W, H) as ctx:
+        ctx.upload(scene)
+
+        def grad(*parts):  # (y, x, tile edge, weight)
+            dL = zero.clone()
+            for y, x, n, w in parts:
+                dL[y:y + n, x:x + n, :3] = w
+            return _plain_gradient(ctx, scene, p, dL)[0, :3].double()
+
+        def lit(x0, w):  # a pixel of the tile whose one path takes the diffuse lobe and meets the sky
+            return next(q for q in ((y, x, 1, w) for y in range(8) for x in range(x0, x0 + 8)) if grad(q)[0] != 0)
+
+        big = lit(0, 2.0 ** 20), lit(32, -2.0 ** 20)
+        small = (512, 0, 8, 2.0 ** -6)
+        ga, gb, gs, g = grad(big[0]), grad(big[1]), grad(small), grad(*big, small)
+    assert torch.all(ga > 2.0 ** 17) and torch.all(gs > 0.1) and torch.all((ga + gb).abs() < 2.0 ** -3 * ga)
+    # g is one rounding to 32 bits of the sum of the three
+    want = ga + gb + gs
+    assert torch.all((g - want).abs() <= 2.0 ** -23 * want.abs() + 0.05 * gs), (g, want, gs)
