@@ -668,7 +668,8 @@ int gk_get_stats(gk_ctx* ctx, gk_stats* out) {
         if (!c.tlas_timed) c.stats.ms_tlas = 0.0;
         else if (hipEventElapsedTime(&a, c.ev[0], c.ev[1]) == hipSuccess) c.stats.ms_tlas = a;
         if (c.timed == Ctx::Timed::stamps) {
-            const unsigned long long* t = words.stamp;
+            unsigned long long t[4] = {words.stamp[0], words.stamp[1], words.stamp[2], 0ull};
+            for (const auto& e : words.end) t[3] = std::max(t[3], e.t);
             int khz = 0;
             GK_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, c.device));
             auto ms = [&](int i, int j) { return t[j] > t[i] ? double(t[j] - t[i]) / double(std::max(khz, 1)) : 0.0; };

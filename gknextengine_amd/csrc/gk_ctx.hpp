@@ -169,10 +169,14 @@ __device__ inline void trace_slot_next(TraceSlot* s) {
 
 // Device words of a context that gk_get_stats reads.
 struct CtxWords {
-    unsigned long long stamp[4];  // clock stamps of the last frame (Ctx::Timed::stamps)
+    unsigned long long stamp[3];  // clock stamps of the last frame (Ctx::Timed::stamps)
     uint32_t single_overflow;     // a stack of the differentiable renderer's traversal overflowed
-    uint32_t pad;
+    uint32_t pad0[25];
+    // the latest end of k_jbf's waves so far, in one of 64 words on lines of their own (the
+    // clock only grows, so a frame's ends are later than those of the frames before)
+    struct { unsigned long long t; uint32_t pad[30]; } end[64];
 };
+static_assert(sizeof(CtxWords) == 128 * 65, "one line each");
 
 // ------------------------------------------------------------------ context
 struct Ctx {
@@ -308,7 +312,8 @@ struct Ctx {
     } wf;
 
     // Stage times of the last frame. Frames with the bilateral post passes: clock stamps by the
-    // kernels themselves (start of the frame, of k_reproject and of k_jbf, end of k_jbf); each
+    // kernels themselves (start of the frame, of k_reproject and of k_jbf, end of k_jbf's last
+    // wave); each
     // event in their place costs 4 to 5 us (16 preview frames at 256x256 with seven each, and a
     // history copy now part of k_jbf: 3.00 -> 2.64 ms). Others, and a TLAS update: events.
     enum class Timed { none, stamps, events, events_no_post } timed = Timed::none;

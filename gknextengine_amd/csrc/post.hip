@@ -40,7 +40,7 @@ struct PostT {
     const uint16_t* moment;
     ushort4* out;
     ushort4 *hist_d, *hist_s, *hist_a;    // k_jbf: the next frame's prev_*
-    unsigned long long* stamp;            // clock stamps (may be null): CtxWords::stamp
+    CtxWords* words;                      // clock stamps (may be null)
 };
 
 // The previous frame's 2x2 footprint at (px, py), with px, py inside the image: element
@@ -101,7 +101,7 @@ __global__ __launch_bounds__(kRB * kRB) void k_reproject(PostK K, PostT T) {
     __shared__ float s_ml[kTileM][kTileM];
     __shared__ float s_kt[25];
     const int tx = int(threadIdx.x), ty = int(threadIdx.y);
-    if (T.stamp && (blockIdx.x | blockIdx.y | threadIdx.x | threadIdx.y) == 0u) T.stamp[1] = wall_clock64();
+    if (T.words && (blockIdx.x | blockIdx.y | threadIdx.x | threadIdx.y) == 0u) T.words->stamp[1] = wall_clock64();
     const int gx = int(blockIdx.x) * kRB, gy = int(blockIdx.y) * kRB;
     const int x = gx + tx, y = gy + ty;
     if (K.progressive) {
@@ -232,7 +232,7 @@ __global__ __launch_bounds__(kJB * kJB) void k_jbf(PostK K, PostT T) {
     // per element here instead of once per tap below
     __shared__ float4 sd[kTile][kTile];
     const int tx = threadIdx.x, ty = threadIdx.y;
-    if (T.stamp && (blockIdx.x | blockIdx.y | threadIdx.x | threadIdx.y) == 0u) T.stamp[2] = wall_clock64();
+    if (T.words && (blockIdx.x | blockIdx.y | threadIdx.x | threadIdx.y) == 0u) T.words->stamp[2] = wall_clock64();
     const int gx = blockIdx.x * kJB, gy = blockIdx.y * kJB;
     const int x = gx + tx, y = gy + ty;
     const f3 lc = f3{0.212671f, 0.715160f, 0.072169f};
@@ -297,9 +297,9 @@ __global__ __launch_bounds__(kJB * kJB) void k_jbf(PostK K, PostT T) {
         K.linear ? to_h4(total.x, total.y, total.z, 1.f)
                  : to_h4(display_encode(total.x, K.paper_white, hdr), display_encode(total.y, K.paper_white, hdr),
                          display_encode(total.z, K.paper_white, hdr), 1.f);
-    // the last work-group to be dispatched
-    if (T.stamp && tx == 0 && ty == 0 && blockIdx.x == gridDim.x - 1u && blockIdx.y == gridDim.y - 1u)
-        T.stamp[3] = wall_clock64();
+    // (a wave's first thread is inside the image if any of its threads is)
+    if (T.words && ((ty * kJB + tx) & 63) == 0)
+        atomicMax(&T.words->end[(blockIdx.y * gridDim.x + blockIdx.x) & 63u].t, (unsigned long long)wall_clock64());
 }
 
 // the learned denoiser's frames: the history, as k_jbf writes it
@@ -361,7 +361,7 @@ int post_process(Ctx& c) {
     T.hist_s = prev_s;
     T.hist_a = prev_a;
     const bool events = c.timed != Ctx::Timed::stamps;
-    T.stamp = events ? nullptr : c.words.ptr->stamp;
+    T.words = events ? nullptr : c.words.ptr;
     if (events) hipEventRecord(c.ev[4], c.stream);
     k_reproject<<<grid, blk, 0, c.stream>>>(K, T);
     GK_HIP(hipGetLastError());

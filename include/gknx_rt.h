@@ -326,7 +326,9 @@ typedef struct gk_stats {
     double ms_shade;           /* raygen + shade + queue compaction/sort       */
     double ms_reproject;
     double ms_denoise;
-    double ms_frame;           /* gk_render, end to end                        */
+    double ms_frame;           /* gk_render's work on the context's stream, from its first kernel
+                                  to the end of its last; ray generation of a frame that follows
+                                  another may start before it, beside the other's last passes */
 } gk_stats;
 
 /* ---------------------------------------------------------------- lifecycle */
