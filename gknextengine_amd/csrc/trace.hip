@@ -172,18 +172,6 @@ __device__ inline float slab1(float lx, float hx, float ly, float hy, float lz, 
     return (hi >= lo && hi >= tmin && lo <= limit) ? lo : __builtin_inff();
 }
 
-// slab test of the 4 children; returns entry distances (or +inf when missed)
-__device__ inline void slab4(const Bvh4Node& n, const Lane& L, float limit, float tl[4]) {
-    const float lx[4] = {n.lox.x, n.lox.y, n.lox.z, n.lox.w};
-    const float hx[4] = {n.hix.x, n.hix.y, n.hix.z, n.hix.w};
-    const float ly[4] = {n.loy.x, n.loy.y, n.loy.z, n.loy.w};
-    const float hy[4] = {n.hiy.x, n.hiy.y, n.hiy.z, n.hiy.w};
-    const float lz[4] = {n.loz.x, n.loz.y, n.loz.z, n.loz.w};
-    const float hz[4] = {n.hiz.x, n.hiz.y, n.hiz.z, n.hiz.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) tl[i] = slab1(lx[i], hx[i], ly[i], hy[i], lz[i], hz[i], L.O, L.rD, L.tmin, limit);
-}
-
 // near_far_offsets: for a direction whose reciprocal component is negative the near plane
 // of that axis is the box's hi plane (offset 16 in the node's lo/hi float4 pair).
 __device__ inline void near_far_offsets(Lane& L) {
@@ -192,7 +180,8 @@ __device__ inline void near_far_offsets(Lane& L) {
     L.sz = (__float_as_uint(L.rD.z) >> 27) & 16u;
 }
 
-// slab4 with the near and far planes fetched by address: per axis, (near - O) * rD and
+// slab test of the 4 children, the near and far planes fetched by address; returns entry
+// distances (or +inf when missed). Per axis, (near - O) * rD and
 // (far - O) * rD are the min and the max of the two plane distances, bit for bit (the
 // rounded difference and the product by a nonzero reciprocal are monotonic, and no term
 // is NaN), so the entry is max3 of the near terms and the exit min3 of the far terms and
@@ -681,7 +670,7 @@ __global__ __launch_bounds__(kBlock) void k_trace(
         // four (distance, entry) pairs go through a fixed 5-exchange sorting network with
         // rejected children at +inf, so every index is static (a variable-length sort
         // compiles to chains of selects on a dynamic index); the accepted children are
-        // then the finite prefix of the sorted four (slab4 returns +inf for a child it
+        // then the finite prefix of the sorted four (slab4_ordered returns +inf for a child it
         // rejects, and accepts only entries <= L.bt). The order of equal distances does
         // not matter: the closest hit is canonical.
         float kt[4];

@@ -59,10 +59,6 @@ __device__ inline bf16x8 ld8(const uint16_t* p) {
 }
 __device__ inline bf16x8 zero8() { return __builtin_bit_cast(bf16x8, make_uint4(0u, 0u, 0u, 0u)); }
 __device__ inline bf16x8 one8() { return __builtin_bit_cast(bf16x8, make_uint4(0x3f80u, 0u, 0u, 0u)); }
-__device__ inline bf16x8 pack8(const uint16_t (&v)[8]) {
-    return __builtin_bit_cast(bf16x8, make_uint4(uint32_t(v[0]) | (uint32_t(v[1]) << 16), uint32_t(v[2]) | (uint32_t(v[3]) << 16),
-                                                 uint32_t(v[4]) | (uint32_t(v[5]) << 16), uint32_t(v[6]) | (uint32_t(v[7]) << 16)));
-}
 // two bf16 gradients where the two bf16 activations are > 0 (sign bit clear and not +0), else 0
 __device__ inline uint32_t relu_mask2(uint32_t gw, uint32_t yw) {
     const uint32_t lo = ((yw & 0x8000u) == 0u && (yw & 0x7fffu) != 0u) ? 0xffffu : 0u;
@@ -1853,7 +1849,6 @@ int launch_wgrad(WgradK K, const WgradPlan& p, hipStream_t st) {
     K.nty = (K.H + th - 1u) / th;
     K.tiles = p.tiles;
     switch (p.mt) {
-        case 4: return launch_wgrad_t<4>(K, p, st);
         case 3: return launch_wgrad_t<3>(K, p, st);
         case 2: return launch_wgrad_t<2>(K, p, st);
         default: return launch_wgrad_t<1>(K, p, st);
