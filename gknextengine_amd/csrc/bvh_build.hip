@@ -535,7 +535,7 @@ __global__ __launch_bounds__(256) void k_collapse(CollapseArgs a, uint32_t level
 // start of the k-th group in order[].
 constexpr uint32_t kCollapseMaxLevels = 255;
 // Primitives of a mesh that one work-group collapses: its 1024 threads then take a level in
-// at most about one round (a level holds at most a quarter of 4096 nodes), 8 to 80 us in all
+// at most two rounds (nodes of a level hold two primitives or more), 8 to 80 us in all
 // against 3 to 5 us for each of about 12 queued levels.
 constexpr uint32_t kCollapseBlockMax = 4096;
 __global__ __launch_bounds__(1024) void k_collapse_block(CollapseArgs a, uint32_t* __restrict__ order,

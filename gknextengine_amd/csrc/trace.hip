@@ -854,7 +854,7 @@ static bool overlap(const void* a, size_t an, const void* b, size_t bn) {
 
 // Whether a launch may read the caller's gk_ray records where they lie: they are aligned for
 // 16-byte loads and no result overwrites a ray that is still to be read. Other rays are copied
-// to a queue first (a pass of 64 bytes a ray: 20 us of 1.15 ms for a million bulk rays).
+// to a queue first (a pass of 64 bytes a ray: 20 us of 1.15 ms for two million bulk rays).
 static bool rays_in_place(const gk_ray* rays, uint32_t n, const gk_hit* hits, const uint32_t* inst) {
     const size_t rb = size_t(n) * sizeof(gk_ray);
     return reinterpret_cast<uintptr_t>(rays) % 16 == 0 && !overlap(rays, rb, hits, size_t(n) * sizeof(gk_hit)) &&

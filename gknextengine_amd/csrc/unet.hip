@@ -1544,7 +1544,9 @@ struct gk_unet {
     DevBuf<float> w32, m, v, grad;
     DevBuf<uint16_t> w16, wt16;
     DevBuf<double> loss;
-    DevBuf<float> wpart;               // partial rows of the weight gradients (training)
+    // partial rows of the weight gradients, from the first training step on: 240 MB for the
+    // 32-channel network (11 MB at 64 x 64 pixels), 64 MB a layer at most but for wider rows
+    DevBuf<float> wpart;
     uint64_t step = 0;
     TensorInfo tinfo[T_COUNT] = {};
     DevBuf<uint16_t> t[T_COUNT];
@@ -1651,7 +1653,10 @@ void launch_conv_m(const ConvK& K, uint32_t nimg, hipStream_t st) {
     // weights join the tile while both stay within 64 KB (two or more work-groups per CU), or
     // whatever fits a CU when the launch has fewer work-groups than CUs: the K loop then waits
     // for no weight load (8 x 256 x 256, input gradients of levels 3 and 4: 21 -> 15 us; at 256
-    // work-groups the copy of the weights costs more than it saves, 21 -> 28 us)
+    // work-groups the copy of the weights costs more than it saves, 21 -> 28 us). Limits of 0,
+    // 96, 128, 192, 255 and none: that step 1033, 1029, 1025, 1022, 1021 and 1057 us; 8 x 384 x
+    // 256 1347, 1344, 1344, 1337, 1339 and 1394; images of 320 x 180 to 1920 x 1080 the same
+    // within 0.5 % up to 255, and up to 7 % longer without a limit
     const uint32_t groups = grid.x * grid.y * grid.z;
     const uint32_t room = groups <= kConvOnePerCu ? max_lds_per_block() : 65536u;
     if (stage && bytes + wbytes <= room) {
@@ -1685,7 +1690,10 @@ int launch_conv(ConvK K, uint32_t nimg, hipStream_t st) {
     // unless the staged input tile is above 64 KB (then every extra work-group stages it
     // again: the level-3 decoder convolution's 86 KB tile at 1080p, 135 tiles, ran at 72 us
     // split three ways against 58 us whole) and there is a tile for every other CU (at 32
-    // tiles, the 8 x 256 x 256 batch: 60 us whole, 31 us split six ways)
+    // tiles, the 8 x 256 x 256 batch: 60 us whole, 31 us split six ways). Inference whole and
+    // split: 15 tiles (640 x 360) 249 and 220 us, 40 (960 x 540) 309 and 277, 60 (1280 x 720)
+    // 449 and 451, 84 545 and 546, 104 621 and 620, 120 749 and 747, 135 777 and 789; training
+    // steps 48 tiles 1367 and 1338 us, 72 1810 and 1792, 96 2188 and 2166, 108 2457 and 2453
     const uint32_t nm = K.cout / 16;
     K.tiles_y = (K.H + 15) / 16;
     const uint32_t tiles = ((K.W + 15) / 16) * K.tiles_y * nimg;
@@ -1806,7 +1814,8 @@ int launch_convs(const gk_unet_layer& L, ConvS K, uint32_t nimg, bool pool, int 
 // each reading the same gradient tile), row groups so that a work-group has about 4 waves, and
 // along the pixels enough work-groups for one per CU: a partial row is as large as the layer's
 // gradient, so more rows cost more to write and add than they hide (step at 192, 256, 384 and
-// 512 work-groups: 1.25, 1.11, 1.16, 1.16 ms). kWgradPart floats of partials at most.
+// 512 work-groups: 1.25, 1.11, 1.16, 1.16 ms). A layer has at most kWgradPart floats of partials,
+// or one row if that is longer; the network keeps those of all layers (gk_unet::wpart).
 constexpr size_t kWgradPart = size_t(1) << 24;
 struct WgradPlan {
     uint32_t mt, ncw, nrg, tiles, rows;  // rows: work-groups along the pixels = partial rows
