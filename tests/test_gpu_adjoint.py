@@ -35,11 +35,16 @@ def setup(W=48, H=48, spp=2, bounces=4):
     return scene, nmat, p
 
 
-def test_primal_matches_oracle_and_adjoint_matches_detached_fd():
+@pytest.mark.parametrize("instances", [1, 2])
+def test_primal_matches_oracle_and_adjoint_matches_detached_fd(instances):
     import torch
     from gknextengine_amd import diff
     W = H = 48
     scene, nmat, p = setup(W, H)
+    if instances == 2:  # the two-level traversal; the second box stands in view, beside the first
+        w = np.diag(np.float32([0.5, 0.5, 0.5, 1.0]))
+        w[:3, 3] = 0.25, 0.1, -0.6
+        scene.add_instance(0, world=w)
     base = list(scene.materials)
     osc = po.OracleScene(scene)
     rng = np.random.default_rng(0)
@@ -233,8 +238,7 @@ def test_descent_recovers_perturbed_parameters_from_an_independent_target():
 
 
 # tiles cut by the image's edge, one to five samples (one, two or four waves on a tile), a
-# single bounce, more bounces than records of all resident paths fit in the record buffer, and
-# a scene of two instances (the two-level traversal)
+# single bounce, many, and a scene of two instances (the two-level traversal)
 @pytest.mark.parametrize("W,H,spp,bounces,instances", [(8, 8, 1, 1, 1), (13, 29, 2, 4, 1), (50, 41, 3, 4, 2),
                                                        (33, 16, 5, 12, 1), (64, 64, 4, 64, 2)])
 def test_shapes_match_oracle_and_single_samples(W, H, spp, bounces, instances):
@@ -414,3 +418,32 @@ def test_sums_of_32_bits_hold_256_pixels():
     # g is one rounding to 32 bits of the sum of the three
     want = ga + gb + gs
     assert torch.all((g - want).abs() <= 2.0 ** -23 * want.abs() + 0.05 * gs), (g, want, gs)
+
+
+# 64-pixel tile groups at four samples, 256-pixel ones at one; 1024 work-groups in one level, 768
+# in two: groups beyond them by a few, and several turns of 256 pixels
+@pytest.mark.parametrize("W,H,spp,bounces,instances", [(264, 264, 4, 4, 1), (520, 520, 1, 3, 1), (768, 701, 1, 3, 2),
+                                                       (224, 232, 4, 4, 2), (800, 600, 4, 2, 1)])
+def test_work_groups_that_take_several_tile_groups(W, H, spp, bounces, instances):
+    """More tile groups than work-groups, so that one uses its records and sums again: the gradient
+    is the sum of gradients whose image derivative is masked to as many groups as work-groups."""
+    import torch
+    scene, nmat, p = setup(W, H, spp, bounces)
+    if instances == 2:
+        w = np.eye(4, dtype=np.float32)
+        w[0, 3] = 1.5
+        scene.add_instance(0, world=w)
+    per = {1: 4, 2: 2, 4: 1}[spp]  # tiles of a group
+    blocks = 1024 if instances == 1 else 768
+    tx, ty = -(-W // 8), -(-H // 8)
+    group = (np.arange(ty)[:, None] * tx + np.arange(tx)[None, :]) // per
+    part = torch.from_numpy(np.kron(group // blocks, np.ones((8, 8), np.int64))[:H, :W]).cuda()
+    assert int(part.max()) >= 1
+    dL = torch.from_numpy(np.random.default_rng(W).normal(size=(H, W, 4)).astype(np.float32)).cuda()
+    with gk.Context(W, H) as ctx:
+        ctx.upload(scene)
+        whole = _plain_gradient(ctx, scene, p, dL)
+        parts = [_plain_gradient(ctx, scene, p, dL * (part == k)[..., None]) for k in range(int(part.max()) + 1)]
+    want = sum(g.double() for g in parts)
+    assert all(float(g.abs().max()) > 0 for g in parts)
+    assert torch.allclose(whole.double(), want, rtol=1e-4, atol=2e-6 * float(want.abs().max())), (whole - want).abs().max()
