@@ -14,7 +14,7 @@ tinybvh BVH::Intersect on host cores.
 
 Other configurations (``--config``): ``dynamic`` (4096 moving instanced bricks,
 TLAS refit every frame, 4 bounces, reprojection + bilateral, 120 frames) and ``cornell``
-(256x256, 16 frames x 1 spp, 4 bounces), ``diff`` (path-replay adjoint
+(256x256, 16 frames x 1 spp, 4 bounces), ``diff`` (adjoint
 at 512x512, 4 spp, with its finite-difference and 4096-spp reference-gradient checks) and
 ``denoise`` (learned vs bilateral denoiser on 1-spp 1080p frames of the city and
 the Cornell box), ``probes`` (the ambient-cube probe grid: voxelize and bake over the
@@ -556,7 +556,7 @@ def denoise_compare(ctx, net, p, ref_spp, reps=20):
 def run_diff(args):
     """Gradient of an L2 image loss with respect to 256 materials x (albedo rgb,
     roughness, metallic) of the tiled Cornell box at 512x512, 4 spp, 4 bounces, by the
-    path-replay adjoint. The target is rendered (256 spp, other seeds) with the parameters
+    adjoint. The target is rendered (256 spp, other seeds) with the parameters
     perturbed by N(0, 0.05). Checks: central differences (h = 1e-3) of the same-seed 4-spp
     loss for albedo (its sampling does not depend on albedo, so the fixed-seed loss is
     smooth in it); a 4096-spp reference gradient (adjoint of the 4096-spp residual); and a
@@ -720,7 +720,7 @@ def run_diff(args):
             "n_gpus": 1, "steps": args.steps, "warmup": 2, "ms_per_step": round(ms, 3), "higher_is_better": False,
             "scaling": "weak", "vs_baseline": None, "dtype": "f32", "data": "synthetic",
             "config": {"workload": "differentiable render: tiled Cornell box, 256 materials x 5 params, "
-                                   "512x512, 4 spp, 4 bounces, L2 loss, path-replay adjoint",
+                                   "512x512, 4 spp, 4 bounces, L2 loss, adjoint",
                        "loss": loss, "paths_per_pass": W * H * spp,
                        "fd_albedo_h1e-3_median_rel_err": float(np.median(fd_err)),
                        "fd_albedo_h1e-3_max_rel_err": float(np.max(fd_err)), "fd_params": len(fd_err),
@@ -992,7 +992,7 @@ def run_diff_timing(args):
     ms = float(np.median(times) * 1e3)
     return {"metric": "forward + adjoint ms", "value": round(ms, 3), "unit": "ms", "steps": args.steps,
             "ms_per_step": round(ms, 3), "higher_is_better": False,
-            "config": {"workload": "differentiable PT_MIS step (512x512, 4 spp): render + L2 loss + path-replay adjoint",
+            "config": {"workload": "differentiable PT_MIS step (512x512, 4 spp): render + L2 loss + adjoint",
                        "resolution": [W, H], "spp": 4, "bounces": 4, "materials": nmat, "params_per_material": 5,
                        "paths_per_step": W * H * 4}}
 

@@ -1,8 +1,8 @@
-// adjoint.hip - differentiable PT_MIS and its path-replay adjoint.
+// adjoint.hip - differentiable PT_MIS and its adjoint.
 //
 // No counterpart in the reference. The primal is the PT_MIS estimator of wavefront.hip
 // (bounded-VNDF GGX + Lambert, NEE to emissive triangles, power-heuristic MIS) without
-// Russian roulette, one thread per pixel, `samples` paths per pixel seeded with pcg4d
+// Russian roulette, `samples` paths per pixel, each by one thread, seeded with pcg4d
 // (x, y, total_frames + s, global_seed); each path starts at a uniformly drawn position
 // inside its pixel (box filter), so image edges and grid-aligned geometry edges are
 // antialiased rather than sampled at one fixed point.
@@ -30,7 +30,8 @@
 // 740 triangles: primal 2.67 ms and adjoint 5.44 ms with one thread per pixel in rows, leaves
 // tested as met, the stack in scratch and every path replayed twice; 2.02 and 2.12 ms with
 // tiles, a wave per sample (the last of 1.3 rounds of resident waves no longer runs four
-// samples) and recorded vertices; 1.04 and 1.25 ms with the traversal of gk_single.hpp.
+// samples) and recorded vertices; 1.04 and 1.25 ms with the traversal of gk_single.hpp (kernel
+// times under the profiler; 0.99 and 1.17 ms queued back to back, with k_reduce_partials).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -341,7 +342,7 @@ __device__ inline void scatter_gradients(const DScene& s, const PathRec& rec, ui
     }
 }
 
-// Four waves per SIMD in single-level scenes (126 registers; at 129, three waves, the primal
+// Four waves per SIMD in single-level scenes (127 registers; at 129, three waves, the primal
 // takes 1.21 ms against 1.04 and the adjoint 1.33 against 1.25), three in two-level ones, whose
 // instance handling would spill.
 template <SingleScene SCENE>

@@ -2,7 +2,8 @@
 
 Parameters are a (num_materials, 5) float32 CUDA tensor: albedo r, g, b, roughness
 (Material.fuzziness), metallic. ``render(params)`` returns the (H, W, 3) radiance image
-(mean of ``samples`` paths per pixel); its backward runs the path-replay adjoint.
+(mean of ``samples`` paths per pixel); its backward runs the adjoint (gk_adjoint), which
+traces the paths again and records their vertices while they are in flight.
 
 The backward replays the materials and frame parameters of its own forward call (not
 whatever the context holds when backward runs), so several renders may precede one

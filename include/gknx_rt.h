@@ -499,11 +499,13 @@ int gk_procgen_brick(float* positions, float* normals, uint32_t* indices, uint32
                      uint32_t* num_vertices, uint32_t* num_triangles);
 
 /* ---------------------------------------------------------------- differentiation
- * Path-replay backpropagation of an image loss with respect to per-material
+ * Backpropagation of an image loss with respect to per-material
  * parameters (albedo rgb, roughness, metalness): 5 floats per material, in
  * material order. No counterpart in the reference (it has no differentiable
- * path). The primal is the PT_MIS estimator at params->samples spp; paths are
- * replayed from their seeds, never stored.
+ * path). The primal is the PT_MIS estimator at params->samples spp and stores no
+ * path; gk_adjoint traces the paths again from their seeds. The context keeps 36
+ * bytes for each vertex that the paths in flight may have: 9.4 MB per bounce of
+ * params->bounces (604 MB at 64), less where the device has not the memory.
  *   d_dl_dimage: device float4 per pixel (dL/d radiance rgb, w ignored)
  *   d_grad:      device 5*num_materials floats, overwritten                    */
 int gk_adjoint(gk_ctx* ctx, const float* d_dl_dimage, float* d_grad);

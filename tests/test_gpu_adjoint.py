@@ -1,4 +1,4 @@
-"""Path-replay adjoint of the differentiable PT_MIS (512x512 Cornell tiles, 256 materials).
+"""Adjoint of the differentiable PT_MIS (512x512 Cornell tiles, 256 materials).
 
 Checks:
   * the GPU primal equals the oracle's double-precision detached render;
